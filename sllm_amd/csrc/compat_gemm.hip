@@ -15,9 +15,10 @@
 // k/bw]. The reference kernel's K-block-major index (fp8.cu:66) contradicts
 // that contract; the contract is what is implemented.
 //
-// These are parity surfaces, not the layer's hot path: a 32x32 LDS-tiled
-// fp32 kernel with on-the-fly dequantization of B (bf16 gemm_ex with
-// k % 128 == 0 takes the MFMA router kernels instead).
+// FP8 and MXFP4 weights of the loader's block shapes run on the matrix cores
+// (gemm_wide.hip), bf16 gemm_ex with k % 128 == 0 on the MFMA router kernels;
+// other shapes take a 32x32 LDS-tiled fp32 kernel with on-the-fly
+// dequantization of B.
 #include "launch.h"
 
 namespace sllm {
@@ -135,6 +136,18 @@ int sllm_fp8_gemm_dev(const float* A, const unsigned char* B,
   SLLM_REQUIRE(M > 0 && N > 0 && K > 0 && block_h > 0 && block_w > 0,
                "sllm_fp8_gemm: bad dims");
   SLLM_REQUIRE(scale_inv, "sllm_fp8_gemm: null scale");
+  // from two rows: the matrix cores (one row: the GEMV below streams B as
+  // fast with less to set up, 8.2 against 8.7 us at 4096 x 4096; two rows
+  // 10.0 against 8.7, 32 rows 76 against 13, 512 rows 738 against 55 on the
+  // tiled kernel). Scale blocks of 4 n rows by 64 2^m columns.
+  const int bws = block_w % 64 == 0 ? __builtin_ctz(block_w / 64) : 0;
+  if (M > 1 && block_w == 64 << bws && block_h % 4 == 0 && A && B && C &&
+      wide_fits(A, B, C, K)) {
+    WideSeg s{};
+    s.a = A; s.total_rows = M; s.w0 = B; s.s0 = scale_inv; s.bh = block_h;
+    s.bws = bws; s.N = N; s.K = K; s.out = C;
+    return launch_wide(WD_FP8, 0, wide_tile(M, N, device_cus()), s, nullptr, 1, nullptr);
+  }
   // decode-size batches with the loader's 128 x 128 blocks: the layer's
   // unpacked-weight GEMV (one wave per four weight rows, 16-byte weight
   // loads dequantized in registers), which streams B once per launch
@@ -197,6 +210,16 @@ int sllm_ds_fp4_gemm_packed_dev(float* o, const float* a, const void* packed,
                                 const void* scale_e8m0, int M, int N, int K,
                                 int block_w) {
   SLLM_REQUIRE(K % 2 == 0 && block_w > 0, "fp4 gemm: K even, block_w > 0");
+  // from two rows: the matrix cores (7168 -> 2048, us: one row 11.9 on the
+  // GEMV below, 14.6 there; four rows 21.9 / 15, 64 rows 286 / 43; 300 rows
+  // 772 on the tiled kernel, 69 there)
+  if (M > 1 && N > 0 && block_w == 32 && a && packed && scale_e8m0 && o &&
+      wide_fits(a, packed, o, K)) {
+    WideSeg s{};
+    s.a = a; s.total_rows = M; s.w0 = (const uint8_t*)packed; s.s0 = scale_e8m0;
+    s.N = N; s.K = K; s.out = o;
+    return launch_wide(WD_FP4, 0, wide_tile(M, N, device_cus()), s, nullptr, 1, nullptr);
+  }
   // decode-size batches with 32-column scale blocks: the layer's
   // unpacked-weight GEMV in its MXFP4 form (the same nibble order, E2M1
   // values and 0x00 / 0xFF scale convention)

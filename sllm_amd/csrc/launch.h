@@ -443,6 +443,37 @@ int launch_gemv(int wf, int swiglu, const void* act, int act_bf16,
                 const void* s0, const uint8_t* w1, const void* s1, int N,
                 int K, const float* row_w, float limit, float* out,
                 hipStream_t st);
+// Unquantized activations against unpacked weights on the matrix cores
+// (gemm_wide.hip): out (fp32) = A . W^T with A fp32, or (swiglu, bf16
+// weights) h = silu(A . w0^T) * (A . w1^T) with A bf16. One or two segments
+// (s1 may be null) of equal format. tile: the workgroup's rows x columns, 0
+// 16 x 16, 1 16 x 32, 2 32 x 64, 3 32 x 128, 4 64 x 128 (swiglu: half the
+// columns of 1-4; wide_tile picks one; tile_info rows must fit). K a
+// multiple of 64 (and 16-byte aligned pointers): wide_fits; FP8: bh a
+// multiple of 4.
+enum { WD_BF16 = 0, WD_FP8 = 1, WD_FP4 = 2 };
+struct WideSeg {
+  const void* a;          // rows, stride K; null: no segment
+  const int* sorted_idx;  // flat assignment index of permuted row p, or null
+  int gather;             // 1: A row of permuted row p is sorted_idx[p] / topk
+  const int* tile_info;   // as SegDesc; null: rows [0, total_rows)
+  const int* num_tiles;
+  int max_tiles, total_rows;
+  const uint8_t* w0;
+  const uint8_t* w1;
+  const void* s0;         // FP8 fp32 / MXFP4 e8m0 scales
+  int bh, bws;            // FP8 scale block: rows of W, log2(K / 64)
+  int N, K;
+  const float* row_w;     // optional: row_w[sorted_idx ? sorted_idx[p] : p]
+  float* out;             // row p, stride N
+};
+int launch_wide(int wf, int swiglu, int tile, const WideSeg& s0,
+                const WideSeg* s1, int topk, hipStream_t st);
+int wide_tile(long rows, long n, int num_cus);
+inline bool wide_fits(const void* a, const void* w, const void* out, int K) {
+  return K % 64 == 0 && (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
+}
+int device_cus();
 int launch_combine(const void* y, int y_f32, const int* inv_pos, int topk,
                    const void* y_shared, int T, int H, int out_f32, void* out,
                    hipStream_t st);

@@ -33,6 +33,7 @@ struct Plan {
   int N;          // T * topk
   int bm, max_tiles;
   int bm_sh;  // decode: rows per tile of the shared expert's launches
+  int wide;   // bf16 weights: the tile of launch_wide
   // decode: K chunks of the streamed gate/up and down launches (routed /
   // shared) and partial-logit slices of the router GEMM
   int ks_up, ks_up_sh, ks_dn, ks_dn_sh, ks_r;
@@ -69,7 +70,16 @@ static int dense8_mode();
 static bool route_inline_on();
 static bool streamk_on();
 static bool split_dealt_on();
-static int device_cus();
+
+// The bf16 layer's tile (launch_wide) for N assignments. 16-row tiles of
+// narrow columns only for the few rows whose launches would leave most CUs
+// idle otherwise; 32 x 128 from there on, also at many rows an expert, where
+// a 64-row tile's second half is mostly padding of an expert's last tile.
+// Layer, us, H 1024 E 16 I 512 top-4 by tile 1 / 2 / 3: 4 assignments 24 /
+// 28 / 34, 16 34 / 30 / 35, 64 44 / 45 / 36, 256 58 / 52 / 42, 4000 394 /
+// 196 / 153 (64 x 128: 143); H 2048 E 32 I 768 top-4: 16 68 / 63 / 52, 4000
+// 811 / 359 / 278 (64 x 128: 291).
+static int bf16_tile(long N) { return N <= 8 ? 1 : (N <= 16 ? 2 : 3); }
 
 static size_t take(size_t& cur, size_t bytes) {
   size_t at = cur;
@@ -109,6 +119,10 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
     // the experts average more than 16 rows (a dense MLP at 17-64 tokens),
     // so that each weight block is streamed once per 32 rows, not per 16
     p.bm = p.N > 16 * std::min(E, p.N) ? 32 : 16;
+    if (force_gemv) {  // bf16 weights: the matrix-core tiles (gemm_wide.hip)
+      p.wide = bf16_tile(p.N);
+      p.bm = p.wide == 1 ? 16 : 32;
+    }
     p.bm_sh = deepseek ? (T > 16 ? 32 : 16) : p.bm;  // Qwen: same launches
   } else {
     p.bm = PREFILL_BM;
@@ -372,6 +386,12 @@ long sllm_moe_qwen_workspace_bytes(const sllm_moe_qwen_args* a) {
 }  // extern "C"
 
 namespace sllm {
+
+// 16-byte aligned bf16 weights and activations (launch_wide's loads).
+static bool wide_weights(const sllm_moe_qwen_args* a) {
+  return wide_fits(a->x, a->wg, a->wu, 64) && wide_fits(a->wd, a->sg, a->su, 64) &&
+         wide_fits(a->sd, nullptr, nullptr, 64);
+}
 
 // The Qwen layer on the workspace ws (ws_bytes bytes): the body of both
 // sllm_moe_qwen_forward (caller's workspace) and
@@ -672,6 +692,32 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
                                             y_sh, T, H, a->out_f32, a->out,
                                             p.ks_dn, (long)p.N * H, p.ks_dn_sh,
                                             (long)T * H, st));
+    } else if (bf16w && wide_weights(a)) {
+      // bf16 weights on the matrix cores, routed and shared segments in one
+      // launch per projection
+      float* h_sh = sh ? (float*)(ws + p.hq_sh) : nullptr;
+      y_sh = sh ? (float*)(ws + p.y_sh) : nullptr;
+      WideSeg r1{}, s1{};
+      r1.a = a->x; r1.sorted_idx = sorted; r1.gather = 1;
+      r1.tile_info = tiles; r1.num_tiles = ntiles; r1.max_tiles = p.max_tiles;
+      r1.w0 = (const uint8_t*)a->wg; r1.w1 = (const uint8_t*)a->wu;
+      r1.N = I; r1.K = H; r1.out = h;
+      s1.a = a->x; s1.total_rows = T;
+      s1.w0 = (const uint8_t*)a->sg; s1.w1 = (const uint8_t*)a->su;
+      s1.N = Is; s1.K = H; s1.out = h_sh;
+      STAGE(clk, SLLM_MOE_STAGE_EXPERT_UP,
+            launch_wide(WD_BF16, 1, p.wide, r1, sh ? &s1 : nullptr, k, st));
+      WideSeg r2{}, s2{};
+      r2.a = h; r2.sorted_idx = sorted;
+      r2.tile_info = tiles; r2.num_tiles = ntiles; r2.max_tiles = p.max_tiles;
+      r2.w0 = (const uint8_t*)a->wd; r2.N = H; r2.K = I; r2.row_w = w; r2.out = y;
+      s2.a = h_sh; s2.total_rows = T;
+      s2.w0 = (const uint8_t*)a->sd; s2.N = H; s2.K = Is; s2.row_w = gate;
+      s2.out = y_sh;
+      STAGE(clk, SLLM_MOE_STAGE_EXPERT_DOWN,
+            launch_wide(WD_BF16, 0, p.wide, r2, sh ? &s2 : nullptr, k, st));
+      STAGE(clk, SLLM_MOE_STAGE_COMBINE,
+            launch_combine(y, 1, inv, k, y_sh, T, H, a->out_f32, a->out, st));
     } else {
     STAGE(clk, SLLM_MOE_STAGE_EXPERT_UP,
           launch_gemv(wf, 1, a->x, 1, 1, sorted, k, p.N, tiles, ntiles,
@@ -1014,7 +1060,7 @@ int sllm_moe_plan_query(int deepseek, int T, int H, int E, int I, int Is,
 
 namespace sllm {
 
-static int device_cus() {
+int device_cus() {
   static int n = 0;
   if (n == 0) {
     int dev = 0;

@@ -1,0 +1,113 @@
+"""The matrix-core kernel over unpacked weights (gemm_wide.hip) at the edges
+of its tiles: FP8 and MXFP4 linears against the fp64 product, the bf16 layer
+against the reference's per-token loop, non-finite activations and scales.
+
+Bound. Every product is exact (an fp32 activation as three bf16 parts); a
+64-wide K step adds at most 6 rounded MFMA sums and one rounded add, and the
+K waves' sums up to 8 more, so |error| <= (7 ceil(K / 64) + 8) 2^-24 sum |a w|,
+plus one rounding of each FP8 scale product."""
+import numpy as np
+import pytest
+
+from oracle import codecs
+from oracle import qwen_moe as qm
+
+pytestmark = pytest.mark.gpu
+
+bf = codecs.round_bf16
+
+
+def _check(got, a, wd):
+    want = a.astype(np.float64) @ wd.astype(np.float64).T
+    mag = np.abs(a).astype(np.float64) @ np.abs(wd).astype(np.float64).T
+    K = a.shape[1]
+    bound = (8 * -(-K // 64) + 8) * 2.0 ** -24 * mag + 1e-30
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
+
+
+# rows at the tiles' edges; columns short of a tile, a scale block or a
+# 16-column subtile; K of one step, of a partial last step over the K waves
+@pytest.mark.parametrize("M", [2, 16, 17, 33, 65, 130])
+@pytest.mark.parametrize("N,K,bh,bw", [(128, 128, 128, 128), (576, 192, 128, 128),
+                                       (133, 64, 4, 64), (40, 1088, 64, 256),
+                                       (2112, 512, 128, 128)])
+def test_fp8_linear(M, N, K, bh, bw):
+    from sllm_amd import fp8
+    rng = np.random.default_rng(M * N + K)
+    a = (rng.standard_normal((M, K)) * 10.0 ** rng.integers(-3, 4, (M, 1))).astype(np.float32)
+    q = rng.integers(0, 256, (N, K), dtype=np.uint8)
+    q[(q & 0x7F) == 0x7F] = 0x30
+    s = (rng.random((-(-N // bh), -(-K // bw))) + 0.5).astype(np.float32)
+    _check(fp8.fp8_gemm(a, q, s, bh, bw), a, codecs.dequant_fp8_block(q, s, (bh, bw)))
+
+
+@pytest.mark.parametrize("M", [2, 17, 65])
+@pytest.mark.parametrize("N,K", [(16, 64), (200, 320), (2048, 1088)])
+def test_fp4_linear(M, N, K):
+    from sllm_amd import deepseek
+    rng = np.random.default_rng(M + N * K)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    s = rng.integers(115, 130, (N, K // 32), dtype=np.uint8)
+    s[0, 0] = 0  # a zero scale
+    _check(deepseek.fp4_moe_linear(a, p, s), a, codecs.dequant_fp4_block(p, s))
+
+
+def test_large_linear_takes_the_tall_tile():
+    from sllm_amd import fp8
+    rng = np.random.default_rng(5)
+    M, N, K = 500, 4100, 256
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    q = rng.integers(0, 0x70, (N, K), dtype=np.uint8)
+    s = (rng.random((-(-N // 128), K // 128)) + 0.5).astype(np.float32)
+    _check(fp8.fp8_gemm(a, q, s), a, codecs.dequant_fp8_block(q, s))
+
+
+@pytest.mark.parametrize("M", [3, 40])
+def test_nonfinite_activations(M):
+    """An infinite activation gives its row's outputs the infinity of its
+    weight's sign, a NaN gives NaN; the other rows and the largest finite
+    value are as without them. A NaN scale gives its output column NaN."""
+    from sllm_amd import deepseek, fp8
+    rng = np.random.default_rng(M)
+    N, K = 96, 256
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    a[0, 5], a[1, 7], a[2, 9] = np.inf, np.nan, np.finfo(np.float32).max
+    q = rng.integers(0x20, 0x30, (N, K), dtype=np.uint8)
+    q[::3] |= 0x80
+    s = np.ones((1, 2), np.float32)
+    got = fp8.fp8_gemm(a, q, s)
+    wd = codecs.dequant_fp8_block(q, s)
+    np.testing.assert_array_equal(got[0], np.where(wd[:, 5] > 0, np.inf, -np.inf))
+    assert np.all(np.isnan(got[1]))
+    _check(got[2:], a[2:], wd)
+    p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    sc = np.full((N, K // 32), 127, np.uint8)
+    sc[4, 1] = 255
+    y = deepseek.fp4_moe_linear(rng.standard_normal((M, K)).astype(np.float32), p, sc)
+    assert np.all(np.isnan(y[:, 4]))
+    assert np.all(np.isfinite(np.delete(y, 4, 1)))
+
+
+@pytest.mark.parametrize("T,k,shared", [(1, 2, True), (5, 3, False), (33, 2, True),
+                                        (70, 4, True), (260, 1, False)])
+def test_bf16_layer_tiles(T, k, shared):
+    """Each tile of the bf16 layer (by assignments: 16-row, 32 x 64, 32 x
+    128), a ragged last row tile, empty experts, with and without the shared
+    segment, against the per-token loop (fp32 there too)."""
+    from sllm_amd.moe import QwenMoE
+    rng = np.random.default_rng(T)
+    H, E, I, Is = 256, 6, 128, 256
+
+    def w(*shape):
+        return bf((rng.standard_normal(shape) * 0.05).astype(np.float32))
+    x = bf(rng.standard_normal((T, H)).astype(np.float32))
+    rw, wg, wu, wd = w(E, H), w(E, I, H), w(E, I, H), w(E, H, I)
+    sg, su, sd, sgl = (w(Is, H), w(Is, H), w(H, Is), w(1, H)) if shared else (None,) * 4
+    layer = QwenMoE(rw, wg, wu, wd, sg=sg, su=su, sd=sd, sgl=sgl, top_k=k)
+    got, r = layer.forward(x, return_routing=True)
+    want = qm.moe_block_grouped(x, r["logits"], wg, wu, wd, k,
+                                (sg, su, sd, sgl) if shared else None)
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    # two chained fp32 products: a few 2^-24 each, the reference's own included
+    assert rel < 2e-6, rel
