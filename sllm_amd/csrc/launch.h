@@ -4,13 +4,15 @@
 
 namespace sllm {
 
-// ks > 1 (T <= 64 only; router_ksplit): the router GEMM writes ks partial
+// ks > 1 (T <= 64 or router_short; router_ksplit): the router GEMM writes ks partial
 // logit slices T * E floats apart, and the routing launches given the same
 // ks add them in order (storing the sum into slice 0). Split, the small
 // router's shared-expert gate is left as ks partial logits at gate_out + T
 // (T floats apart); a softmax routing launch given that buffer as gate
 // adds them in order and writes the sigmoid to gate[0, T).
 int router_ksplit(int T, int H);
+int router_one_round(int H);
+bool router_short(int T, int E);
 // Prefill (T > 64) may also zero zero_n ints at zero: the permutation's
 // chunk histograms, which a softmax routing launch given them as
 // chunk_hist then fills (integer atomics: the counts do not depend on

@@ -53,6 +53,8 @@ struct Plan {
                 // then the fused combine's (fcnt_on)
   bool fcnt_on;
   size_t rpart;  // Qwen prefill router partials (RouterPart), or 0
+  size_t rlog;   // the router's K slices of a short prompt (in the y rows), or 0
+  int ks_l;      // partial-logit slices that the routing launch reads
   size_t total;
 };
 
@@ -280,6 +282,17 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
     p.y = take(c, (size_t)p.N * H * 2);                       // y bf16
     p.y_sh = has_shared ? take(c, (size_t)T * H * 2) : 0;
   }
+  // A short prompt's router slices lie in the y rows, which the down launch
+  // writes after the routing launch has read them.
+  p.ks_l = p.ks_r;
+  if (need_logits && router_short(T, E)) {
+    const size_t yb = p.decode ? (size_t)p.ks_dn * p.N * H * 4 : (size_t)p.N * H * 2;
+    const int ks = router_one_round(H);
+    if (ks > 1 && (size_t)ks * T * E * 4 <= yb) {
+      p.rlog = p.y;
+      p.ks_l = ks;
+    }
+  }
   p.total = c;
   return p;
 }
@@ -343,6 +356,14 @@ static int check_common(const A* a, const char* who) {
   return 0;
 }
 
+static int copy_logits(float* out, const float* logits, int T, int E,
+                       hipStream_t st) {
+  if (out)
+    SLLM_HIP(hipMemcpyAsync(out, logits, (size_t)T * E * 4,
+                            hipMemcpyDeviceToDevice, st));
+  return 0;
+}
+
 static int copy_debug(const float* logits, const float* w, const int* ids,
                       const int* counts, const int* sorted, const int* inv,
                       int T, int E, int N, float* logits_out, float* w_out,
@@ -353,9 +374,7 @@ static int copy_debug(const float* logits, const float* w, const int* ids,
                             hipMemcpyDeviceToDevice, st));
   if (inv_out)
     SLLM_HIP(hipMemcpyAsync(inv_out, inv, (size_t)N * 4, hipMemcpyDeviceToDevice, st));
-  if (logits_out)
-    SLLM_HIP(hipMemcpyAsync(logits_out, logits, (size_t)T * E * 4,
-                            hipMemcpyDeviceToDevice, st));
+  if (copy_logits(logits_out, logits, T, E, st)) return -1;
   if (w_out)
     SLLM_HIP(hipMemcpyAsync(w_out, w, (size_t)N * 4, hipMemcpyDeviceToDevice, st));
   if (ids_out)
@@ -418,7 +437,8 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
                "sllm_moe_qwen_forward: workspace %ld < %zu bytes", ws_bytes,
                p.total);
   hipStream_t st = (hipStream_t)a->stream;
-  float* logits = a->logits_given ? (float*)a->logits : (float*)(ws + p.logits);
+  float* logits = a->logits_given ? (float*)a->logits
+                                  : (float*)(ws + (p.rlog ? p.rlog : p.logits));
   float* w = (float*)(ws + p.w);
   int* ids = (int*)(ws + p.ids);
   int* counts = (int*)(ws + p.counts);
@@ -535,7 +555,7 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
   // activations and forms partial shared-expert gates from the x tiles it
   // holds; the routing launch merges the partials.
   const bool topk_router = !small_router && !one_expert && !small_route &&
-                           !a->logits_given && p.rpart != 0;
+                           !a->logits_given && p.rpart != 0 && !router_short(T, E);
   RouterPart rp{};
   if (topk_router) {
     rp = router_part_at(ws + p.rpart, T, E, k);
@@ -557,7 +577,7 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
                                    rp, st, chunk_hist, hist_n)
               : launch_router_gemm((const uint16_t*)a->x,
                                    (const uint16_t*)a->router_w, logits, T, E,
-                                   H, st, 1, chunk_hist, hist_n));
+                                   H, st, p.ks_l, chunk_hist, hist_n));
   }
   if (one_expert || route_inl) {
     STAGE(clk, SLLM_MOE_STAGE_ROUTE, 0);
@@ -575,10 +595,11 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
     STAGE(clk, SLLM_MOE_STAGE_ROUTE,
           topk_router
               ? launch_route_merge(rp, T, E, eps, w, ids, st, chunk_hist)
-              : launch_route_softmax(logits, w, ids, T, E, k, eps, st, p.ks_r,
+              : launch_route_softmax(logits, w, ids, T, E, k, eps, st, p.ks_l,
                                      gate_fin, chunk_hist,
                                      aq_fused ? &aq : nullptr,
                                      a->router_bias));
+    if (p.rlog && copy_logits(a->logits_out, logits, T, E, st)) return -1;
     STAGE(clk, SLLM_MOE_STAGE_PERMUTE,
           perm_inl ? 0
                    : launch_permute(ids, p.N, E, p.bm, counts, offsets, sorted,
@@ -853,7 +874,8 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
   }
   if (clk.finish()) return -1;
   return copy_debug(logits, w, ids, counts, sorted, inv, T, E, p.N,
-                    a->logits_out, a->w_out, a->ids_out, a->counts_out,
+                    p.rlog ? nullptr : a->logits_out, a->w_out, a->ids_out,
+                    a->counts_out,
                     a->sorted_out, a->inv_pos_out, st);
 }
 
@@ -1145,7 +1167,8 @@ int sllm_moe_ds_forward(const sllm_moe_ds_args* a) {
                a->workspace_bytes, p.total);
   hipStream_t st = (hipStream_t)a->stream;
   char* ws = (char*)a->workspace;
-  float* logits = a->logits_given ? (float*)a->logits : (float*)(ws + p.logits);
+  float* logits = a->logits_given ? (float*)a->logits
+                                  : (float*)(ws + (p.rlog ? p.rlog : p.logits));
   float* w = (float*)(ws + p.w);
   int* ids = (int*)(ws + p.ids);
   int* counts = (int*)(ws + p.counts);
@@ -1160,7 +1183,7 @@ int sllm_moe_ds_forward(const sllm_moe_ds_args* a) {
   // scales) from the x chunks it stages, in place of the activation-quant
   // launch, which would read x again (C4: 117 MB).
   const bool rq_fused = !p.decode && !a->logits_given &&
-                        router_logits_quant_fits(T, H);
+                        !router_short(T, E) && router_logits_quant_fits(T, H);
   // Streamed decode up to RI_MAX_ROUTE_T tokens with the router launch: the
   // routed gate/up launch also routes the batch (grouped scoring, a token
   // per wave, in every workgroup), in place of the routing launch; the
@@ -1198,16 +1221,17 @@ int sllm_moe_ds_forward(const sllm_moe_ds_args* a) {
                                        fcnt, nfcnt + nccnt)
             : launch_router_gemm((const uint16_t*)a->x,
                                  (const uint16_t*)a->router_w, logits, T, E,
-                                 H, st, p.ks_r));
+                                 H, st, p.ks_l));
   STAGE(clk, SLLM_MOE_STAGE_ROUTE,
         route_inl ? 0
         : a->tid2eid
             ? launch_route_hash(logits, a->token_ids, a->tid2eid, a->vocab, w,
                                 ids, T, E, k, a->scoring, a->route_scale, st,
-                                p.ks_r)
+                                p.ks_l)
             : launch_route_grouped(logits, a->bias, w, ids, T, E, k,
                                    a->n_group, a->topk_group, a->scoring,
-                                   a->route_scale, st, p.ks_r));
+                                   a->route_scale, st, p.ks_l));
+  if (p.rlog && copy_logits(a->logits_out, logits, T, E, st)) return -1;
   // Streamed decode otherwise: the routed gate/up launch builds the
   // permutation from the routing launch's ids in every workgroup
   // (RouteInline.ids_in), in place of the permutation launch, as in the
@@ -1453,7 +1477,8 @@ int sllm_moe_ds_forward(const sllm_moe_ds_args* a) {
   }
   if (clk.finish()) return -1;
   return copy_debug(logits, w, ids, counts, sorted, inv, T, E, p.N,
-                    a->logits_out, a->w_out, a->ids_out, a->counts_out,
+                    p.rlog ? nullptr : a->logits_out, a->w_out, a->ids_out,
+                    a->counts_out,
                     a->sorted_out, a->inv_pos_out, st);
 }
 

@@ -165,8 +165,8 @@ __global__ __launch_bounds__(512, 1) void router_gemm_kernel(
       }
 }
 
-// Small T (decode, T <= 64): a workgroup owns 16 experts and all T tokens;
-// its 8 waves split K (wave w takes the 32-wide slices w, w + 8, ...) so the
+// Small T (decode, T <= 64; the few token tiles of a short prompt): a
+// workgroup owns 16 experts and up to 64 tokens (tile blockIdx.z); its 8 waves split K (wave w takes the 32-wide slices w, w + 8, ...) so the
 // router weights stream through many CUs at once; partial sums are reduced
 // through LDS.
 constexpr int RG_SMALL_T = 64;
@@ -190,11 +190,13 @@ __global__ __launch_bounds__(512) void router_gemm_small_kernel(
     int* __restrict__ zero, long nzero) {
   __shared__ float part[8][NTI * 16][16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (long i = ((long)blockIdx.y * gridDim.x + blockIdx.x) * 512 + threadIdx.x;
-       i < nzero; i += (long)gridDim.x * gridDim.y * 512)
+  for (long i = (((long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 512 +
+                threadIdx.x;
+       i < nzero; i += (long)gridDim.x * gridDim.y * gridDim.z * 512)
     zero[i] = 0;
   const int lr = lane & 15, lg = lane >> 4;
   const int e0 = blockIdx.x * 16;
+  const int t0 = blockIdx.z * RG_SMALL_T, tn = min(RG_SMALL_T, T - t0);
   const bool gate_tile = e0 >= E;
   const int nsl = H / 32, ks = gridDim.y, q = blockIdx.y;
   const int s0 = q * nsl / ks, s1 = (q + 1) * nsl / ks;
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(512) void router_gemm_small_kernel(
   const uint16_t* arow[NTI];
 #pragma unroll
   for (int i = 0; i < NTI; ++i)
-    arow[i] = x + (size_t)min(i * 16 + lr, T - 1) * H + lg * 8;
+    arow[i] = x + (size_t)(t0 + min(i * 16 + lr, tn - 1)) * H + lg * 8;
   f32x4 acc[NTI];
 #pragma unroll
   for (int i = 0; i < NTI; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -232,8 +234,8 @@ __global__ __launch_bounds__(512) void router_gemm_small_kernel(
 #pragma unroll
     for (int v = 0; v < 4; ++v) part[wave][i * 16 + lg * 4 + v][lr] = acc[i][v];
   __syncthreads();
-  float* out = logits + (size_t)q * T * E;
-  for (int qq = threadIdx.x; qq < T * 16; qq += 512) {
+  float* out = logits + (size_t)q * T * E + (size_t)t0 * E;
+  for (int qq = threadIdx.x; qq < tn * 16; qq += 512) {
     const int r = qq >> 4, c = qq & 15;
     float s = 0.f;
 #pragma unroll
@@ -845,6 +847,23 @@ static int epl_for(int E) {
 // CUs rather than T / 4 (the reads are bound by per-CU bandwidth).
 static int route_tokens_per_block(int ks) { return ks > 1 ? 1 : 4; }
 
+// Prompts whose 64-token x 128-expert tiles (the fused prefill router's)
+// would leave most CUs idle, each tile walking K alone behind two chunks in
+// flight: 24 us at 333 tokens x 512 experts x H 2048 (24 workgroups), 7168
+// wide 3.5 times that. They take the decode router's kernel instead (16
+// experts x 64 tokens, K over eight waves and the workgroups' K chunks), then
+// the softmax or grouped routing over its slices, which also quantizes the
+// activations (Qwen; DeepSeek by the activation-quant launch). Layer, us,
+// fused -> this, by tiles: E 512 H 2048 T 65 (8 tiles) 225 -> 217, 333 (24)
+// 314 -> 309, 512 (32) 322 -> 318, 768 (48) 329 -> 331, 1024 (64) 336 -> 343;
+// E 128 T 200 (4) 150 -> 131, 2048 (32) 252 -> 244; E 64 H 3072 T 75 (2)
+// 228 -> 198, 2048 (32) 385 -> 370; DeepSeek E 256 H 7168 T 200 (8) 1121 ->
+// 1081, 1024 (32) 1326 -> 1322, 2048 (64) 1584 -> 1622.
+constexpr int RG_SHORT_TILES = 32;
+bool router_short(int T, int E) {
+  return T > RG_SMALL_T && ceil_div(T, RG_TT) * ceil_div(E, RG_TE) <= RG_SHORT_TILES;
+}
+
 // K chunks of the decode router: at least two, and enough that each of a
 // workgroup's 8 waves takes at most four 32-wide K slices, one round of
 // loads in flight together. H = 2048 (C3): 2, as every further slice costs
@@ -852,11 +871,13 @@ static int route_tokens_per_block(int ks) { return ks > 1 ? 1 : 4; }
 // 155-157 us, 2 chunks 153-155, 4 chunks 153-156, 8 chunks 156-157).
 // H = 7168 (C4): 7; two chunks left each wave four rounds of loads (the
 // router 8.9 us at B=1), and 8 chunks took C4 decode B=1 / 8 / 32 from
-// 98 / 281 / 680 to 94 / 274 / 672 us.
+// 98 / 281 / 680 to 94 / 274 / 672 us. Short prompts (router_short)
+// take the one round (router_one_round).
+int router_one_round(int H) { return (H / 32 + 31) / 32; }
+
 int router_ksplit(int T, int H) {
   if (T > RG_SMALL_T) return 1;
-  const int one_round = (H / 32 + 31) / 32;
-  return std::max(std::max(1, std::min(2, H / 256)), one_round);
+  return std::max(std::max(1, std::min(2, H / 256)), router_one_round(H));
 }
 
 static int launch_router_small(const uint16_t* x, const uint16_t* w,
@@ -866,7 +887,8 @@ static int launch_router_small(const uint16_t* x, const uint16_t* w,
                                long nzero = 0) {
   SLLM_REQUIRE(ks >= 1 && ks <= H / 32, "router_small: bad K split %d", ks);
   SLLM_REQUIRE(nzero >= 0 && (nzero == 0 || zero), "router_small: bad zero range");
-  const dim3 grid(ceil_div(E, 16) + (gate_out ? 1 : 0), ks);
+  SLLM_REQUIRE(!gate_out || T <= RG_SMALL_T, "router_small: gate needs T <= %d", RG_SMALL_T);
+  const dim3 grid(ceil_div(E, 16) + (gate_out ? 1 : 0), ks, ceil_div(T, RG_SMALL_T));
 #define CASE(n)                                                              \
   router_gemm_small_kernel<n><<<grid, 512, 0, st>>>(x, w, logits, T, E, H,   \
                                                     sgl, gate_out, zero, nzero)
@@ -888,12 +910,12 @@ int launch_router_gemm(const uint16_t* x, const uint16_t* w, float* logits,
   SLLM_REQUIRE(T > 0 && E > 0 && H > 0 && H % 128 == 0,
                "router_gemm: need T,E>0 and H %% 128 == 0 (T=%d E=%d H=%d)",
                T, E, H);
-  SLLM_REQUIRE(ks == 1 || T <= RG_SMALL_T, "router_gemm: K split needs T <= %d",
-               RG_SMALL_T);
-  SLLM_REQUIRE(zero_n == 0 || (zero && T > RG_SMALL_T),
-               "router_gemm: zeroing needs the prefill kernel");
-  if (T <= RG_SMALL_T) {
-    return launch_router_small(x, w, logits, T, E, H, nullptr, nullptr, ks, st);
+  const bool small = T <= RG_SMALL_T || router_short(T, E);
+  SLLM_REQUIRE(ks == 1 || small, "router_gemm: K split of T=%d E=%d", T, E);
+  SLLM_REQUIRE(zero_n == 0 || zero, "router_gemm: null zero range");
+  if (small) {
+    return launch_router_small(x, w, logits, T, E, H, nullptr, nullptr, ks, st,
+                               zero, zero_n);
   } else {
     dim3 grid(ceil_div(T, RG_TT), ceil_div(E, RG_TE));
     router_gemm_kernel<<<grid, 512, 0, st>>>(x, w, logits, T, E, H, zero,
