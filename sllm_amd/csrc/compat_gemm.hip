@@ -146,7 +146,7 @@ int sllm_fp8_gemm_dev(const float* A, const unsigned char* B,
     WideSeg s{};
     s.a = A; s.total_rows = M; s.w0 = B; s.s0 = scale_inv; s.bh = block_h;
     s.bws = bws; s.N = N; s.K = K; s.out = C;
-    return launch_wide(WD_FP8, 0, wide_tile(M, N, device_cus()), s, nullptr, 1, nullptr);
+    return launch_wide(WD_FP8, 0, wide_tile(WD_FP8, M, N, device_cus()), s, nullptr, 1, nullptr);
   }
   // decode-size batches with the loader's 128 x 128 blocks: the layer's
   // unpacked-weight GEMV (one wave per four weight rows, 16-byte weight
@@ -218,7 +218,7 @@ int sllm_ds_fp4_gemm_packed_dev(float* o, const float* a, const void* packed,
     WideSeg s{};
     s.a = a; s.total_rows = M; s.w0 = (const uint8_t*)packed; s.s0 = scale_e8m0;
     s.N = N; s.K = K; s.out = o;
-    return launch_wide(WD_FP4, 0, wide_tile(M, N, device_cus()), s, nullptr, 1, nullptr);
+    return launch_wide(WD_FP4, 0, wide_tile(WD_FP4, M, N, device_cus()), s, nullptr, 1, nullptr);
   }
   // decode-size batches with 32-column scale blocks: the layer's
   // unpacked-weight GEMV in its MXFP4 form (the same nibble order, E2M1

@@ -29,10 +29,11 @@
 // What bounds it: vector ALU issue beside the MFMAs (the split, 5
 // instructions an element, is repeated by every column tile; the FP8
 // conversion one per two weights), two waves a SIMD. FP8 512 x 4096 x 4096:
-// 738 us on the tiled kernel, 55-58 here (0.9 PFLOP/s of bf16 products, the
+// 738 us on the tiled kernel, 56 here (0.9 PFLOP/s of bf16 products, the
 // product itself 300 TFLOP/s); 32 rows 76 -> 13 us. MXFP4 300 x 2048 x 7168:
 // 772 -> 69 us. bf16 layer (H 1024, E 16, I 512, top-4): 64 tokens 212 -> 42
-// us, 1000 tokens 2712 -> 153 us. Against 64 bits the error is that of the
+// us, 1000 tokens 2712 -> 115 us, there by the L2's rate: a tile's K step
+// brings its rows of both operands in (32 x 128 tiles: 153 us). Against 64 bits the error is that of the
 // GEMV (1.1e-7 to 1.6e-7) and below the tiled kernel's (1.1e-6, 1.4e-6).
 #include "launch.h"
 
@@ -429,23 +430,30 @@ int go(const WideSeg& s0, const WideSeg& s1, int topk, hipStream_t st) {
 
 }  // namespace
 
-// The tiles (rows x output columns) and the time of one of their workgroups
-// in us on FP8 weights at K = 4096, by which wide_tile weighs them.
-static const struct { int bm, bn; float us; } WIDE_TILE[] = {
-    {16, 16, 12.f}, {16, 32, 12.9f}, {32, 64, 22.f}, {32, 128, 30.f}, {64, 128, 54.f}};
+// The linears' tiles (rows x output columns) and the time of one of their
+// workgroups in us at K = 4096, FP8 and MXFP4 weights, by which wide_tile
+// weighs them.
+struct WideTile {
+  int bm, bn;
+  float us;
+};
+static const WideTile WIDE_FP8[] = {
+    {16, 16, 12.f}, {16, 32, 12.7f}, {32, 64, 23.f}, {32, 128, 33.5f}, {32, 256, 53.f}};
+static const WideTile WIDE_FP4[] = {
+    {16, 16, 9.5f}, {16, 32, 12.5f}, {32, 64, 23.8f}, {32, 128, 39.f}, {64, 128, 64.f}};
 
 // One workgroup fits a CU (its registers and tile), so a launch takes as
-// many rounds as its tiles need over the CUs. FP8 4096 x 4096, us by tile
-// (16x16 / 16x32 / 32x64 / 32x128 / 64x128): 16 rows 12.0 / 12.9 / 23 / 30 /
-// 54, 32 rows 21.5 / 13.2 / 23 / 31 / 55, 128 rows - / - / 26 / 32 / 56, 256
-// rows - / - / 47 / 33 / 56, 512 rows - / - / 91 / 62 / 58.
-int wide_tile(long rows, long n, int num_cus) {
+// many rounds as its tiles need over the CUs. FP8 4096 x 4096, us by tile:
+// 16 rows 11.8 / 12.4 / 23 / 34 / 54, 32 rows 21.7 / 12.7 / 23 / 34 / 55, 256
+// rows - / - / 50 / 36 / 55, 512 rows - / - / 93 / 68 / 56 (64 x 128, which
+// spills there: 62; MXFP4's tallest, where 32 x 256 takes 13% longer).
+int wide_tile(int wf, long rows, long n, int num_cus) {
+  const WideTile* tile = wf == WD_FP8 ? WIDE_FP8 : WIDE_FP4;
   int best = 0;
   float t = 0.f;
   for (int i = 0; i < 5; ++i) {
-    const auto& w = WIDE_TILE[i];
-    const long tiles = (rows + w.bm - 1) / w.bm * ((n + w.bn - 1) / w.bn);
-    const float c = w.us * (float)((tiles + num_cus - 1) / num_cus);
+    const long tiles = (rows + tile[i].bm - 1) / tile[i].bm * ((n + tile[i].bn - 1) / tile[i].bn);
+    const float c = tile[i].us * (float)((tiles + num_cus - 1) / num_cus);
     if (i == 0 || c < t) {
       best = i;
       t = c;
@@ -458,20 +466,21 @@ int launch_wide(int wf, int swiglu, int tile, const WideSeg& s0,
                 const WideSeg* s1, int topk, hipStream_t st) {
   const WideSeg z{};
   const WideSeg& t1 = s1 ? *s1 : z;
-#define GO(WF_)                                                            \
+#define GO(WF_, BM4_, WN4_)                                                \
   (tile == 0   ? go<WF_, true, false, 16, 1, 1>(s0, t1, topk, st)          \
    : tile == 1 ? go<WF_, true, false, 16, 1, 2>(s0, t1, topk, st)          \
    : tile == 2 ? go<WF_, true, false, 32, 2, 2>(s0, t1, topk, st)          \
    : tile == 3 ? go<WF_, true, false, 32, 4, 2>(s0, t1, topk, st)          \
-               : go<WF_, true, false, 64, 4, 2>(s0, t1, topk, st))
-  if (wf == WD_FP8) return GO(WD_FP8);
-  if (wf == WD_FP4) return GO(WD_FP4);
+               : go<WF_, true, false, BM4_, WN4_, 2>(s0, t1, topk, st))
+  if (wf == WD_FP8) return GO(WD_FP8, 32, 8);
+  if (wf == WD_FP4) return GO(WD_FP4, 64, 4);
 #undef GO
 #define GO(A_, SW_)                                                        \
   (tile == 1   ? go<WD_BF16, A_, SW_, 16, 1, 2>(s0, t1, topk, st)          \
    : tile == 2 ? go<WD_BF16, A_, SW_, 32, 2, 2>(s0, t1, topk, st)          \
-               : go<WD_BF16, A_, SW_, 32, 4, 2>(s0, t1, topk, st))
-  SLLM_REQUIRE(tile >= 1 && tile <= 3, "wide gemm: tile %d of bf16 weights", tile);
+   : tile == 3 ? go<WD_BF16, A_, SW_, 32, 4, 2>(s0, t1, topk, st)          \
+               : go<WD_BF16, A_, SW_, 64, 8, 2>(s0, t1, topk, st))
+  SLLM_REQUIRE(tile >= 1 && tile <= 4, "wide gemm: tile %d of bf16 weights", tile);
   return swiglu ? GO(false, true) : GO(true, false);
 #undef GO
 }

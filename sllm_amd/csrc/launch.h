@@ -449,8 +449,9 @@ int launch_gemv(int wf, int swiglu, const void* act, int act_bf16,
 // (gemm_wide.hip): out (fp32) = A . W^T with A fp32, or (swiglu, bf16
 // weights) h = silu(A . w0^T) * (A . w1^T) with A bf16. One or two segments
 // (s1 may be null) of equal format. tile: the workgroup's rows x columns, 0
-// 16 x 16, 1 16 x 32, 2 32 x 64, 3 32 x 128, 4 64 x 128 (swiglu: half the
-// columns of 1-4; wide_tile picks one; tile_info rows must fit). K a
+// 16 x 16, 1 16 x 32, 2 32 x 64, 3 32 x 128, 4 32 x 256 (FP8), 64 x 128
+// (MXFP4) or 64 x 256 (bf16); swiglu: half the columns of 1-4; wide_tile
+// picks the linears'; tile_info rows must fit. K a
 // multiple of 64 (and 16-byte aligned pointers): wide_fits; FP8: bh a
 // multiple of 4.
 enum { WD_BF16 = 0, WD_FP8 = 1, WD_FP4 = 2 };
@@ -471,7 +472,7 @@ struct WideSeg {
 };
 int launch_wide(int wf, int swiglu, int tile, const WideSeg& s0,
                 const WideSeg* s1, int topk, hipStream_t st);
-int wide_tile(long rows, long n, int num_cus);
+int wide_tile(int wf, long rows, long n, int num_cus);
 inline bool wide_fits(const void* a, const void* w, const void* out, int K) {
   return K % 64 == 0 && (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
 }

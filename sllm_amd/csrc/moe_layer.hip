@@ -73,15 +73,21 @@ static bool route_inline_on();
 static bool streamk_on();
 static bool split_dealt_on();
 
-// The bf16 layer's tile (launch_wide) for N assignments. 16-row tiles of
-// narrow columns only for the few rows whose launches would leave most CUs
-// idle otherwise; 32 x 128 from there on, also at many rows an expert, where
-// a 64-row tile's second half is mostly padding of an expert's last tile.
-// Layer, us, H 1024 E 16 I 512 top-4 by tile 1 / 2 / 3: 4 assignments 24 /
-// 28 / 34, 16 34 / 30 / 35, 64 44 / 45 / 36, 256 58 / 52 / 42, 4000 394 /
-// 196 / 153 (64 x 128: 143); H 2048 E 32 I 768 top-4: 16 68 / 63 / 52, 4000
-// 811 / 359 / 278 (64 x 128: 291).
-static int bf16_tile(long N) { return N <= 8 ? 1 : (N <= 16 ? 2 : 3); }
+// The bf16 layer's tile (launch_wide) for N assignments of T tokens. 16-row
+// tiles of narrow columns only for the few rows whose launches would leave
+// most CUs idle otherwise, 32 x 128 from there on, 64 x 256 (half the weight
+// bytes an output) once the experts hold 24 rows and such tiles half the
+// CUs. Layer, us, H 1024 E 16 I 512 top-4 by tile 1 / 2 / 3 / 4: 4
+// assignments 24 / 28 / 34 / -, 16 34 / 30 / 35 / -, 64 44 / 45 / 36 / 50, 256
+// 58 / 52 / 42 / 59, 1000 - / 72 / 67 / 66, 2000 - / 118 / 90 / 70, 4000 394 /
+// 196 / 155 / 115; H 2048 E 32 I 768 top-4: 64 113 / 99 / 95 / 92, 512 - / -
+// / 105 / 106, 1000 - / 152 / 131 / 113, 4000 811 / 359 / 284 / 213.
+static int bf16_tile(long N, long E, long T, long I, bool has_shared) {
+  if (N <= 16) return N <= 8 ? 1 : 2;
+  const long m = std::min(E, N), r = N / m;
+  const long tiles = (N + 32 * m) / 64 + (has_shared ? (T + 63) / 64 : 0);
+  return r >= 24 && tiles * (I / 128) >= device_cus() / 2 ? 4 : 3;
+}
 
 static size_t take(size_t& cur, size_t bytes) {
   size_t at = cur;
@@ -122,8 +128,8 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
     // so that each weight block is streamed once per 32 rows, not per 16
     p.bm = p.N > 16 * std::min(E, p.N) ? 32 : 16;
     if (force_gemv) {  // bf16 weights: the matrix-core tiles (gemm_wide.hip)
-      p.wide = bf16_tile(p.N);
-      p.bm = p.wide == 1 ? 16 : 32;
+      p.wide = bf16_tile(p.N, E, T, I, has_shared);
+      p.bm = p.wide == 1 ? 16 : (p.wide < 4 ? 32 : 64);
     }
     p.bm_sh = deepseek ? (T > 16 ? 32 : 16) : p.bm;  // Qwen: same launches
   } else {

@@ -90,10 +90,11 @@ def test_nonfinite_activations(M):
 
 
 @pytest.mark.parametrize("T,k,shared", [(1, 2, True), (5, 3, False), (33, 2, True),
-                                        (70, 4, True), (260, 1, False)])
+                                        (70, 4, True), (260, 1, False),
+                                        (2900, 3, True), (1701, 5, False)])
 def test_bf16_layer_tiles(T, k, shared):
     """Each tile of the bf16 layer (by assignments: 16-row, 32 x 64, 32 x
-    128), a ragged last row tile, empty experts, with and without the shared
+    128, 64 x 256), a ragged last row tile, empty experts, with and without the shared
     segment, against the per-token loop (fp32 there too)."""
     from sllm_amd.moe import QwenMoE
     rng = np.random.default_rng(T)
