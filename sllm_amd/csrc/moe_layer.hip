@@ -149,7 +149,8 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
   p.ntiles = take(c, 4);
   p.pscr = take(c, permute_scratch_bytes(p.N, E));
   // shared-expert gate, then (split router) its ks_r partial slices
-  p.gate = take(c, (size_t)(p.ks_r > 1 ? 1 + p.ks_r : 1) * T * 4);
+  const int ks_g = p.decode && T > DECODE_MAX_T ? router_one_round(H) : p.ks_r;
+  p.gate = take(c, (size_t)(ks_g > 1 ? 1 + ks_g : 1) * T * 4);
   if (!deepseek && !p.decode && need_logits && router_topk_fits(T, E, topk, H))
     p.rpart = take(c, router_part_bytes(T, E, topk));
   if (p.decode) {
@@ -480,7 +481,12 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
   // (B=8: 76.5 vs 76.9 us with the fused finish). A stream-K gate/up
   // launch (every unit in K slices) finishes in the launch at any decode
   // batch whose router launch clears the counters.
-  const bool small_router = p.decode && !a->logits_given && T <= 64;
+  // (above 64 tokens, the bf16 layer's prompts: the same launch, with the
+  // gate in it, while one workgroup permutes the batch; larger batches keep
+  // the launch that clears the permutation's histograms)
+  const bool small_router = p.decode && !a->logits_given &&
+                            (T <= 64 || (router_short(T, E) && bf16w &&
+                                         !permute_uses_chunk_hist(p.N, E)));
   const bool fused = p.decode && a->wgu_packed && !one_expert && !bf16w &&
                      p.fcnt_on && (p.ks_up > 1 || p.ks_up_sh > 1) &&
                      (T <= DEC_FUSE_MAX_T || (p.sk_up && small_router));
@@ -540,12 +546,12 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
           launch_router_small_gate((const uint16_t*)a->x,
                                    (const uint16_t*)a->router_w, logits, T, E,
                                    H, sh ? (const uint16_t*)a->sgl : nullptr,
-                                   sh ? gate : nullptr, st, p.ks_r,
+                                   sh ? gate : nullptr, st, p.ks_l,
                                    rzero, nrzero));
     gate_done = sh;
   }
   // split router: the routing launch finishes the gate from its partials
-  float* gate_fin = small_router && sh && p.ks_r > 1 ? gate : nullptr;
+  float* gate_fin = small_router && sh && p.ks_l > 1 ? gate : nullptr;
   // Prefill router GEMM + softmax routing + multi-workgroup permutation: the
   // router zeroes the permutation's chunk histograms and the routing launch
   // fills them, which saves the permutation's histogram launch.

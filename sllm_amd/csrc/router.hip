@@ -242,8 +242,8 @@ __global__ __launch_bounds__(512) void router_gemm_small_kernel(
     for (int wv = 0; wv < 8; ++wv) s += part[wv][r][c];
     if (gate_tile) {
       if (c == 0) {
-        if (ks == 1) gate_out[r] = sigmoid_f32(s);
-        else gate_out[T + q * T + r] = s;
+        if (ks == 1) gate_out[t0 + r] = sigmoid_f32(s);
+        else gate_out[T + q * T + t0 + r] = s;
       }
     } else if (e0 + c < E) {
       out[(size_t)r * E + e0 + c] = s;
@@ -887,7 +887,6 @@ static int launch_router_small(const uint16_t* x, const uint16_t* w,
                                long nzero = 0) {
   SLLM_REQUIRE(ks >= 1 && ks <= H / 32, "router_small: bad K split %d", ks);
   SLLM_REQUIRE(nzero >= 0 && (nzero == 0 || zero), "router_small: bad zero range");
-  SLLM_REQUIRE(!gate_out || T <= RG_SMALL_T, "router_small: gate needs T <= %d", RG_SMALL_T);
   const dim3 grid(ceil_div(E, 16) + (gate_out ? 1 : 0), ks, ceil_div(T, RG_SMALL_T));
 #define CASE(n)                                                              \
   router_gemm_small_kernel<n><<<grid, 512, 0, st>>>(x, w, logits, T, E, H,   \
@@ -1034,7 +1033,8 @@ int launch_router_small_gate(const uint16_t* x, const uint16_t* w,
                              float* logits, int T, int E, int H,
                              const uint16_t* sgl, float* gate_out,
                              hipStream_t st, int ks, int* zero, long nzero) {
-  SLLM_REQUIRE(x && w && logits && T > 0 && T <= RG_SMALL_T && E > 0 &&
+  SLLM_REQUIRE(x && w && logits && T > 0 && E > 0 &&
+                   (T <= RG_SMALL_T || router_short(T, E)) &&
                    H % 32 == 0 && (!gate_out || sgl),
                "router_small_gate: bad args (T=%d E=%d H=%d)", T, E, H);
   return launch_router_small(x, w, logits, T, E, H, sgl, gate_out, ks, st,

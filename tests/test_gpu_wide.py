@@ -89,16 +89,19 @@ def test_nonfinite_activations(M):
     assert np.all(np.isfinite(np.delete(y, 4, 1)))
 
 
-@pytest.mark.parametrize("T,k,shared", [(1, 2, True), (5, 3, False), (33, 2, True),
-                                        (70, 4, True), (260, 1, False),
-                                        (2900, 3, True), (1701, 5, False)])
-def test_bf16_layer_tiles(T, k, shared):
+@pytest.mark.parametrize("T,k,shared,H", [
+    (1, 2, True, 256), (5, 3, False, 256), (33, 2, True, 256), (70, 4, True, 256),
+    (260, 1, False, 256), (2900, 3, True, 256), (1701, 5, False, 256),
+    (90, 2, True, 2048), (200, 3, True, 1280)])
+def test_bf16_layer_tiles(T, k, shared, H):
     """Each tile of the bf16 layer (by assignments: 16-row, 32 x 64, 32 x
     128, 64 x 256), a ragged last row tile, empty experts, with and without the shared
-    segment, against the per-token loop (fp32 there too)."""
+    segment, against the per-token loop (fp32 there too). Above 64 tokens the
+    router's launch also forms the shared gate: in one K chunk, or (H 1280,
+    2048) in two partials."""
     from sllm_amd.moe import QwenMoE
     rng = np.random.default_rng(T)
-    H, E, I, Is = 256, 6, 128, 256
+    E, I, Is = 6, 128, 256
 
     def w(*shape):
         return bf((rng.standard_normal(shape) * 0.05).astype(np.float32))
