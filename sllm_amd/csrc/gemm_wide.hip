@@ -29,8 +29,8 @@
 // What bounds it: vector ALU issue beside the MFMAs (the split, 5
 // instructions an element, is repeated by every column tile; the FP8
 // conversion one per two weights), two waves a SIMD. FP8 512 x 4096 x 4096:
-// 738 us on the tiled kernel, 56 here (0.9 PFLOP/s of bf16 products, the
-// product itself 300 TFLOP/s); 32 rows 76 -> 13 us. MXFP4 300 x 2048 x 7168:
+// 738 us on the tiled kernel, 54 here (0.95 PFLOP/s of bf16 products, the
+// product itself 317 TFLOP/s); 32 rows 76 -> 13 us. MXFP4 300 x 2048 x 7168:
 // 772 -> 69 us. bf16 layer (H 1024, E 16, I 512, top-4): 64 tokens 212 -> 42
 // us, 1000 tokens 2712 -> 115 us, there by the L2's rate: a tile's K step
 // brings its rows of both operands in (32 x 128 tiles: 153 us). Against 64 bits the error is that of the
@@ -438,15 +438,20 @@ struct WideTile {
   float us;
 };
 static const WideTile WIDE_FP8[] = {
-    {16, 16, 12.f}, {16, 32, 12.7f}, {32, 64, 23.f}, {32, 128, 33.5f}, {32, 256, 53.f}};
+    {16, 16, 12.f}, {16, 32, 12.7f}, {32, 64, 23.f}, {32, 128, 33.5f}, {32, 256, 50.f}};
 static const WideTile WIDE_FP4[] = {
     {16, 16, 9.5f}, {16, 32, 12.5f}, {32, 64, 23.8f}, {32, 128, 39.f}, {64, 128, 64.f}};
 
 // One workgroup fits a CU (its registers and tile), so a launch takes as
 // many rounds as its tiles need over the CUs. FP8 4096 x 4096, us by tile:
 // 16 rows 11.8 / 12.4 / 23 / 34 / 54, 32 rows 21.7 / 12.7 / 23 / 34 / 55, 256
-// rows - / - / 50 / 36 / 55, 512 rows - / - / 93 / 68 / 56 (64 x 128, which
-// spills there: 62; MXFP4's tallest, where 32 x 256 takes 13% longer).
+// rows - / - / 50 / 36 / 55, 512 rows - / - / 93 / 68 / 54 (64 x 128, which
+// spills there: 62). The tallest FP8 tile is four waves of 64 columns by two
+// K halves: an LDS fragment serves four products, not two, and half as many
+// barriers follow (eight waves of 32 columns: 300 / 400 / 512 rows 54.7 / 55.9 /
+// 57.4 us, so 51.3 / 51.9 / 54.1). MXFP4, whose conversions that form holds
+// in registers too, keeps 64 x 128 (7168 <- 2048, 150 / 222 / 512 rows 37.3 /
+// 38.4 / 76.0 us there, 44.0 / 44.9 / 88.1 as 32 x 256).
 int wide_tile(int wf, long rows, long n, int num_cus) {
   const WideTile* tile = wf == WD_FP8 ? WIDE_FP8 : WIDE_FP4;
   int best = 0;
@@ -466,14 +471,14 @@ int launch_wide(int wf, int swiglu, int tile, const WideSeg& s0,
                 const WideSeg* s1, int topk, hipStream_t st) {
   const WideSeg z{};
   const WideSeg& t1 = s1 ? *s1 : z;
-#define GO(WF_, BM4_, WN4_)                                                \
+#define GO(WF_, BM4_, WN4_, NC4_)                                          \
   (tile == 0   ? go<WF_, true, false, 16, 1, 1>(s0, t1, topk, st)          \
    : tile == 1 ? go<WF_, true, false, 16, 1, 2>(s0, t1, topk, st)          \
    : tile == 2 ? go<WF_, true, false, 32, 2, 2>(s0, t1, topk, st)          \
    : tile == 3 ? go<WF_, true, false, 32, 4, 2>(s0, t1, topk, st)          \
-               : go<WF_, true, false, BM4_, WN4_, 2>(s0, t1, topk, st))
-  if (wf == WD_FP8) return GO(WD_FP8, 32, 8);
-  if (wf == WD_FP4) return GO(WD_FP4, 64, 4);
+               : go<WF_, true, false, BM4_, WN4_, NC4_>(s0, t1, topk, st))
+  if (wf == WD_FP8) return GO(WD_FP8, 32, 4, 4);
+  if (wf == WD_FP4) return GO(WD_FP4, 64, 4, 2);
 #undef GO
 #define GO(A_, SW_)                                                        \
   (tile == 1   ? go<WD_BF16, A_, SW_, 16, 1, 2>(s0, t1, topk, st)          \

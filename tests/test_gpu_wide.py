@@ -53,13 +53,15 @@ def test_fp4_linear(M, N, K):
     _check(deepseek.fp4_moe_linear(a, p, s), a, codecs.dequant_fp4_block(p, s))
 
 
-def test_large_linear_takes_the_tall_tile():
+# two whole 128-wide K steps; a half last step, which one K wave sits out
+@pytest.mark.parametrize("K", [256, 320])
+def test_large_linear_takes_the_tall_tile(K):
     from sllm_amd import fp8
     rng = np.random.default_rng(5)
-    M, N, K = 500, 4100, 256
+    M, N = 500, 4100
     a = rng.standard_normal((M, K)).astype(np.float32)
     q = rng.integers(0, 0x70, (N, K), dtype=np.uint8)
-    s = (rng.random((-(-N // 128), K // 128)) + 0.5).astype(np.float32)
+    s = (rng.random((-(-N // 128), -(-K // 128))) + 0.5).astype(np.float32)
     _check(fp8.fp8_gemm(a, q, s), a, codecs.dequant_fp8_block(q, s))
 
 
