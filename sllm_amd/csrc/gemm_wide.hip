@@ -19,10 +19,10 @@
 // Tile. Eight waves; a workgroup owns BM rows (16, 32 or 64) and WN waves'
 // columns, each NC 16-column subtiles wide; the other 8 / WN split every K
 // step, so that a few rows still keep eight waves' weight loads in flight
-// and the K loop short; their sums meet in LDS at the end, added in wave
-// order. Activations go through LDS (bf16 planes, double buffered, one
-// barrier a step, split once per workgroup); weights go straight to the wave
-// that multiplies them, three K steps ahead, in the K order that makes a
+// and the K loop short; their sums meet in LDS at the end, added pairwise.
+// Activations go through LDS (bf16 planes, double buffered, one barrier a
+// step, split once per workgroup); weights go straight to the wave that
+// multiplies them, three K steps ahead, in the K order that makes a
 // lane's load 16 or 32 contiguous bytes (lane group g takes K [16 g, +16) of
 // a 64-wide step for both operands).
 //
@@ -31,10 +31,12 @@
 // conversion one per two weights), two waves a SIMD. FP8 512 x 4096 x 4096:
 // 738 us on the tiled kernel, 54 here (0.95 PFLOP/s of bf16 products, the
 // product itself 317 TFLOP/s); 32 rows 76 -> 13 us. MXFP4 300 x 2048 x 7168:
-// 772 -> 69 us. bf16 layer (H 1024, E 16, I 512, top-4): 64 tokens 212 -> 42
-// us, 1000 tokens 2712 -> 115 us, there by the L2's rate: a tile's K step
-// brings its rows of both operands in (32 x 128 tiles: 153 us). Against 64 bits the error is that of the
-// GEMV (1.1e-7 to 1.6e-7) and below the tiled kernel's (1.1e-6, 1.4e-6).
+// 772 -> 69 us. bf16 layer (H 1024, E 16, I 512, top-4): 64 tokens 212 -> 43
+// us, 1000 tokens 2712 -> 110 us, there by the L2's rate: a tile's K step
+// brings its rows of both operands in (32 x 128 tiles: 153 us). Against 64
+// bits the error is below that of the GEMV (layer 1.5e-7 to 1.8e-7 up to 64
+// tokens) and of the tiled kernel (linears 1.3e-7 and 1.6e-7, there 1.1e-6 and
+// 1.4e-6).
 #include "launch.h"
 
 namespace sllm {
@@ -136,6 +138,13 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   constexpr int NA = BM * KT / CE / WD_THREADS;  // such chunks per thread
   constexpr int NW = WBytes<WF>::regs;
   static_assert(NA >= 1 && NA * CE * WD_THREADS == BM * KT, "whole chunks");
+  // gate/up up to 32-row tiles: the K steps' sum keeps its rounding errors
+  // beside it. Layer against 64 bits at 64 tokens, H 1024 / 2048: 1.64e-7 /
+  // 1.98e-7 without (the GEMV 1.60e-7 / 1.82e-7), 1.48e-7 / 1.69e-7 with it, for 1
+  // to 3% of the layer's time (41.9 -> 42.9 us, 104 -> 106); in the down launch
+  // too 1.46e-7 / 1.64e-7 for twice that. 64-row tiles are below the GEMV that
+  // they replaced without it (1.82e-7 against 1.84e-7, 2.3e-7 against 3.6e-7).
+  constexpr bool COMP = SWIGLU && BM <= 32;
   constexpr int TILE = PL * BM * LS;  // elements of one step's tile
   constexpr int RED = WK > 1 ? (8 - WN) * RB * NC * 64 * 8 : 0;  // (bf16 sized)
   // (two arrays: a step's reads of one cannot alias its writes of the other)
@@ -241,6 +250,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   for (int r = 0; r < RB; ++r)
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[r][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  f32x4 low[COMP ? RB : 1][COMP ? NC : 1] = {};
 
   uint32_t m1lo = 0x0000BF80u;  // bf16 (-1, 0), kept in a register
   asm("" : "+v"(m1lo));
@@ -301,6 +311,11 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int v = 0; v < 4; ++v)
+          if constexpr (COMP) {
+            const float a0 = acc[r][c][v], p0 = part[r][c][v], t = a0 + p0;
+            low[r][c][v] += p0 - (t - a0);
+            acc[r][c][v] = t;
+          } else
           acc[r][c][v] = WF == WD_FP8 ? fmaf(part[r][c][v], cur.f[c], acc[r][c][v])
                                       : acc[r][c][v] + part[r][c][v];
   };
@@ -365,6 +380,16 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   rest(a_lds0, a_lds1, t2, t3);
   rest(a_lds1, a_lds0, t3, t0);
 
+  if constexpr (COMP) {  // (past an infinity the lost part is a NaN)
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (__builtin_isfinite(acc[r][c][v])) acc[r][c][v] += low[r][c][v];
+  }
+
   // ---- the K waves' sums ----------------------------------------------------
   if constexpr (WK > 1) {
     f32x4* red = (f32x4*)a_lds0;
@@ -377,12 +402,21 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
     }
     __syncthreads();
     if (wk > 0) return;
-    for (int k = 1; k < WK; ++k)
 #pragma unroll
-      for (int r = 0; r < RB; ++r)
+    for (int r = 0; r < RB; ++r)
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-          acc[r][c] += red[(((k - 1) * WN + wn) * RB * NC + r * NC + c) * 64 + lane];
+      for (int c = 0; c < NC; ++c) {
+        f32x4 t[WK];
+        t[0] = acc[r][c];
+#pragma unroll
+        for (int k = 1; k < WK; ++k)
+          t[k] = red[(((k - 1) * WN + wn) * RB * NC + r * NC + c) * 64 + lane];
+#pragma unroll
+        for (int d = 1; d < WK; d *= 2)
+#pragma unroll
+          for (int k = 0; k < WK; k += 2 * d) t[k] += t[k + d];
+        acc[r][c] = t[0];
+      }
   }
   // ---- epilogue: lane = token r * 16 + lc, columns 4 lg + v of a subtile ----
 #pragma unroll
