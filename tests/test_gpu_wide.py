@@ -117,3 +117,23 @@ def test_bf16_layer_tiles(T, k, shared, H):
     rel = np.linalg.norm(got - want) / np.linalg.norm(want)
     # two chained fp32 products: a few 2^-24 each, the reference's own included
     assert rel < 2e-6, rel
+
+
+@pytest.mark.parametrize("T", [3, 40])
+def test_bf16_layer_infinity(T):
+    """An infinite activation under positive weights leaves its token
+    infinite, not NaN through the compensated sum; the others as without."""
+    from sllm_amd.moe import QwenMoE
+    rng = np.random.default_rng(T)
+    E, I, H, k = 4, 128, 1024, 2
+
+    def w(*shape):
+        return bf((rng.random(shape) * 0.05 + 0.01).astype(np.float32))
+    x = bf(rng.standard_normal((T, H)).astype(np.float32))
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    layer = QwenMoE(w(E, H), w(E, I, H), w(E, I, H), w(E, H, I), top_k=k)
+    want = layer.forward(x, logits=logits)
+    x[0, 5] = np.inf
+    got = layer.forward(x, logits=logits)
+    assert np.all(got[0] == np.inf)
+    np.testing.assert_array_equal(got[1:], want[1:])
