@@ -125,6 +125,49 @@ __device__ __forceinline__ bf16x8 w_frag(const uint32_t* r, int m, uint32_t sb) 
   }
 }
 
+// Row n of weight block e against the fp32 row a by plain fp32 products, the
+// weight scaled first, by a whole wave (each lane 16 values of every 1024).
+template <int WF>
+__device__ float plain_dot(const WideSeg& S, const float* a, int e, int n, int lane) {
+  const int K = S.K;
+  const size_t row = (size_t)e * S.N + n;
+  float sum = 0.f;
+  for (int k = 16 * lane; k < K; k += 1024) {
+    float w[16], d = 0.f;
+    if constexpr (WF == WD_FP8) {
+      const uint4 q = *(const uint4*)(S.w0 + row * K + k);
+      const uint32_t b[4] = {q.x, q.y, q.z, q.w};
+      const float s = ((const float*)S.s0)[(size_t)(n / S.bh) * ((K + (64 << S.bws) - 1) >> (6 + S.bws)) +
+                                           (k >> (6 + S.bws))];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) w[i] = e4m3_to_f32(b[i / 4], i & 3) * s;
+    } else {
+      bf16x8 h[2];
+      if constexpr (WF == WD_FP4) {
+        const uint2 q = *(const uint2*)(S.w0 + row * (K / 2) + k / 2);
+        const uint32_t sb = ((const uint8_t*)S.s0)[row * (K / 32) + k / 32];
+        h[0] = e2m1x8(q.x, sb);
+        h[1] = e2m1x8(q.y, sb);
+      } else {
+        h[0] = *(const bf16x8*)(S.w0 + (row * K + k) * 2);
+        h[1] = *(const bf16x8*)(S.w0 + (row * K + k) * 2 + 16);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) w[i] = (float)h[i / 8][i % 8];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      const float4 v = *(const float4*)(a + k + i);
+      d = fmaf(v.x, w[i], d);
+      d = fmaf(v.y, w[i + 1], d);
+      d = fmaf(v.z, w[i + 2], d);
+      d = fmaf(v.w, w[i + 3], d);
+    }
+    sum += d;
+  }
+  return wave_sum(sum);
+}
+
 template <int WF, bool A32, bool SWIGLU, int BM, int WN, int NC>
 __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1,
                                                           int blocks0, int topk) {
@@ -441,6 +484,39 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
 #pragma unroll
         for (int v = 0; v < 4; ++v)
           if (n + v < N) d[v] = o[v];
+      }
+    }
+  }
+  // An infinite or NaN sum of fp32 activations may be this kernel's own: an
+  // FP8 partial that overflows before a small block scale, or an infinite
+  // weight (a bf16 one, e8m0 254) against a zero mid or lo part. Those
+  // outputs are taken again by plain fp32 products, an output at a time by
+  // the whole wave (its weights laid out as the loads above read them).
+  if constexpr (A32) {
+    static_assert(RB * NC * 4 <= 32, "a bit for each of a lane's sums");
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < RB * NC * 4; ++i)
+      z = fmaf(acc[i / (4 * NC)][i / 4 % NC][i % 4], 0.f, z);
+    if (!__ballot(z != 0.f)) return;
+    uint32_t bad = 0;
+#pragma unroll
+    for (int i = 0; i < RB * NC * 4; ++i) {
+      const int r = i / (4 * NC), c = i / 4 % NC, v = i % 4;
+      if (r * 16 + lc < rows && ncol + c * 16 + 4 * lg + v < N &&
+          !__builtin_isfinite(acc[r][c][v]))
+        bad |= 1u << i;
+    }
+    while (const uint64_t m = __ballot(bad != 0)) {
+      const int l = __builtin_ctzll(m);
+      const int i = __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)bad, l));
+      const int t = i / (4 * NC) * 16 + (l & 15), p = rb0 + t;
+      const int n = ncol + i / 4 % NC * 16 + 4 * (l >> 4) + i % 4;
+      float y = plain_dot<WF>(S, (const float*)S.a + (size_t)rsrc[t] * K, e, n, lane);
+      if (S.row_w) y *= S.row_w[S.sorted_idx ? S.sorted_idx[p] : p];
+      if (lane == l) {
+        S.out[(size_t)p * N + n] = y;
+        bad &= bad - 1;
       }
     }
   }

@@ -91,6 +91,72 @@ def test_nonfinite_activations(M):
     assert np.all(np.isfinite(np.delete(y, 4, 1)))
 
 
+def _product(a, wd):
+    """The fp64 product with what 0 and infinities give (an fp32 overflow as
+    an infinity)."""
+    with np.errstate(all="ignore"):
+        return (a.astype(np.float64)[:, None, :] * wd.astype(np.float64)[None]).sum(-1) \
+            .astype(np.float32)
+
+
+@pytest.mark.parametrize("M", [3, 40, 260])
+def test_fp8_linear_block_scale_range(M):
+    """Activations whose products with the unscaled codes overflow: the block
+    scale belongs to the weight, so a small one keeps the result finite, a
+    zero one makes it 0, an infinite one infinite (NaN beside a zero code)."""
+    from sllm_amd import fp8
+    rng = np.random.default_rng(M)
+    N, K = 520, 256
+    a = (rng.standard_normal((M, K)) + 2.0).astype(np.float32) * np.float32(1e36)
+    a[1] = 1.0  # exact in bf16: nothing in its two lower parts
+    q = rng.integers(0x70, 0x7F, (N, K), dtype=np.uint8)
+    q[::2, ::3] |= 0x80
+    s = np.full((5, 2), 1e-3, np.float32)
+    s[1] = 0.0
+    s[2, 1] = np.inf
+    q[260:300, 130] = 0
+    got = fp8.fp8_gemm(a, q, s)
+    wd = codecs.dequant_fp8_block(q, s)
+    finite = np.r_[0:256, 384:N]
+    _check(got[:, finite], a, wd[finite])
+    assert np.all(got[:, 128:256] == 0)
+    np.testing.assert_array_equal(got[:, 256:384], _product(a, wd[256:384]))
+
+
+@pytest.mark.parametrize("M", [2, 40])
+def test_infinite_weights(M):
+    """An infinite weight (e8m0 254; a bf16 one in the down projection) gives
+    its outputs the infinity of the product's sign, as a plain product does,
+    also where the activation is exact in bf16."""
+    from sllm_amd import deepseek
+    from sllm_amd.moe import QwenMoE
+    rng = np.random.default_rng(M)
+    N, K = 48, 128
+    a = rng.integers(1, 5, (M, K)).astype(np.float32)
+    p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    p[:, 16:32] = 0
+    p[:, 16] = 0x44  # twice 2, times 2^127 where the scale is 254
+    s = np.full((N, K // 32), 127, np.uint8)
+    s[::2, 1] = 254
+    got = deepseek.fp4_moe_linear(a, p, s)
+    assert np.all(np.isposinf(got[:, ::2]))
+    _check(got[:, 1::2], a, codecs.dequant_fp4_block(p, s)[1::2])
+
+    E, I, H, T = 2, 128, 256, 3 * M
+    w = lambda *n: bf((rng.standard_normal(n) * 0.05).astype(np.float32))  # noqa: E731
+    x, rw, wg, wu, wd = bf(rng.standard_normal((T, H)).astype(np.float32)), w(E, H), \
+        w(E, I, H), w(E, I, H), w(E, H, I)
+    wu[:, 5] = 0  # h = 0 there: NaN against an infinite weight
+    wd[0, 7, 9], wd[1, 11, 3], wd[0, 20, 5] = np.inf, -np.inf, np.inf
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    got = QwenMoE(rw, wg, wu, wd, top_k=1).forward(x, logits=logits)
+    with np.errstate(all="ignore"):
+        want = qm.moe_block_grouped(x, logits, wg, wu, wd, 1, None)
+    fin = np.isfinite(want)
+    np.testing.assert_array_equal(got[~fin], want[~fin])
+    np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("T,k,shared,H", [
     (1, 2, True, 256), (5, 3, False, 256), (33, 2, True, 256), (70, 4, True, 256),
     (260, 1, False, 256), (2900, 3, True, 256), (1701, 5, False, 256),
