@@ -8,8 +8,9 @@
 // (decode.hip), which multiplies on the vector ALU and passes over the
 // weights once per four rows, is not bound by the weight stream any more.
 //
-// fp32 precision on bf16 MFMAs. An fp32 activation is the exact sum of three
-// bf16 values, its significand cut in 8 + 8 + 8 bits (split3), and every
+// fp32 precision on bf16 MFMAs. An fp32 activation, times a power of two, is
+// the exact sum of three bf16 values, its significand cut in 8 + 8 + 8 bits
+// (split3), and every
 // weight format here is exact in bf16 (FP8 before its block scale), so the
 // three products per weight are exact and are added in fp32: the arithmetic
 // of an fp32 dot product, in another order. bf16 activations (x) need one
@@ -67,15 +68,23 @@ __device__ __forceinline__ void sub_bf16(float& v0, float& v1, uint32_t p,
   v1 = __builtin_amdgcn_fdot2_f32_bf16(q, __builtin_bit_cast(bf16x2, 0xBF800000u), v1, false);
 }
 
-// Two fp32 values as three bf16 pairs each cut off (truncated) in turn:
-// hi + mid + lo is the value exactly (8 + 8 + 8 significand bits). An
-// infinity is the hi part's, with finite mid and lo; a quiet NaN is hi's.
+// fp32 activations are multiplied by 2^A_UP before they are cut, and the sums
+// by 2^-A_UP at the end: bf16's smallest step is 2^-133, and v_dot2_f32_bf16
+// drops results below 2^-126, so that unscaled the mid and lo parts of values
+// below 2^-109 lost bits (2^-118: 2e-5 off, 2^-130: 7%). Scaled, every fp32
+// value keeps all of them.
+constexpr int A_UP = 40;
+
+// Two fp32 values, scaled, as three bf16 pairs each cut off (truncated) in
+// turn: hi + mid + lo is the value exactly (8 + 8 + 8 significand bits). An
+// infinity or NaN, or a value past 2^88, gives its row's sums infinities or
+// NaN, which are taken again.
 __device__ __forceinline__ void split3(float a, float b, uint32_t m1lo,
                                        uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = pack_hi(a, b);
-  constexpr float F = 3.402823466e38f;
-  float ra = __builtin_amdgcn_fmed3f(a, -F, F), rb = __builtin_amdgcn_fmed3f(b, -F, F);
-  sub_bf16(ra, rb, pack_hi(ra, rb), m1lo);
+  constexpr float UP = (float)(1ull << A_UP);
+  float ra = a * UP, rb = b * UP;
+  hi = pack_hi(ra, rb);
+  sub_bf16(ra, rb, hi, m1lo);
   mid = pack_hi(ra, rb);
   sub_bf16(ra, rb, mid, m1lo);
   lo = pack_hi(ra, rb);
@@ -375,6 +384,11 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
       constexpr int U = PL * RB;
       constexpr int VALU = (A32 ? 20 * NA : 0) + (WF == WD_BF16 ? 0 : 8 * NC) + 4 * RB * NC;
       constexpr int V = VALU / (2 * U) > 0 ? VALU / (2 * U) : 1;
+      // the second half's share, where another one measured better: FP8 32 x
+      // 256 (fewer registers live: 62 us at 512 x 4096 x 4096 with V, 54 so),
+      // 32-row tiles over MXFP4 (300 x 2048 x 7168 70.0 -> 66.6) and bf16
+      // weights (the layer's down launch, 64 tokens: -0.3)
+      constexpr int V2 = NC == 4 ? V - 4 : A32 && WF != WD_FP8 && BM == 32 ? V + 2 : V;
       __builtin_amdgcn_sched_group_barrier(0x100, U, 0);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -385,7 +399,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         __builtin_amdgcn_sched_group_barrier(0x008, NC, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, V2, 0);
       }
     }
     __syncthreads();
@@ -462,6 +476,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
       }
   }
   // ---- epilogue: lane = token r * 16 + lc, columns 4 lg + v of a subtile ----
+  constexpr float DOWN = A32 ? 1.f / (float)(1ull << A_UP) : 1.f;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
     const int t = r * 16 + lc;
@@ -476,7 +491,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
 #pragma unroll
       for (int v = 0; v < 4; ++v)
         o[v] = SWIGLU ? silu_f32(acc[r][c][v]) * acc[r][c + (SWIGLU ? NO : 0)][v]
-                      : acc[r][c][v] * w;
+                      : acc[r][c][v] * DOWN * w;
       float* d = S.out + (size_t)p * N + n;
       if (n + 4 <= N && N % 4 == 0) {
         *(float4*)d = make_float4(o[0], o[1], o[2], o[3]);

@@ -123,6 +123,26 @@ def test_fp8_linear_block_scale_range(M):
     np.testing.assert_array_equal(got[:, 256:384], _product(a, wd[256:384]))
 
 
+@pytest.mark.parametrize("M", [3, 40])
+@pytest.mark.parametrize("e", [-112, -124, -136])
+def test_tiny_activations(M, e):
+    """Activations near and below fp32's smallest normal value keep their
+    bits: the result is a plain fp32 product's to its rounding."""
+    from sllm_amd import deepseek, fp8
+    rng = np.random.default_rng(M - e)
+    N, K = 96, 256
+    a = np.ldexp(rng.standard_normal((M, K)), e).astype(np.float32)
+    q = rng.integers(0, 0x70, (N, K), dtype=np.uint8)
+    s = np.full((1, 2), 2.0 ** 60, np.float32)
+    p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    sc = np.full((N, K // 32), 127 + 60, np.uint8)
+    for got, wd in ((fp8.fp8_gemm(a, q, s), codecs.dequant_fp8_block(q, s)),
+                    (deepseek.fp4_moe_linear(a, p, sc), codecs.dequant_fp4_block(p, sc))):
+        mag = np.abs(a).astype(np.float64) @ np.abs(wd).astype(np.float64).T
+        err = np.abs(got - a.astype(np.float64) @ wd.astype(np.float64).T)
+        assert np.all(err <= (8 * (K // 64) + 8) * 2.0 ** -24 * mag), np.max(err / mag)
+
+
 @pytest.mark.parametrize("M", [2, 40])
 def test_infinite_weights(M):
     """An infinite weight (e8m0 254; a bf16 one in the down projection) gives
