@@ -13,9 +13,9 @@
 // waves owns 4 weight rows per wave; lane l reads 16-byte chunks
 // l, l+64, ... of each row (coalesced 1 KB per wave instruction), converts
 // them with the gfx950 fp8/fp4 conversions and accumulates dot products
-// against up to 4 activation rows at a time; a wave reduction finishes each
-// dot. gemv1 pairs gate row n with up row n in the same wave so SwiGLU is
-// applied before anything leaves registers.
+// against up to 4 activation rows at a time; a wave reduction in 64 bits
+// finishes each dot. gemv1 pairs gate row n with up row n in the same wave so
+// SwiGLU is applied before anything leaves registers.
 #include "launch.h"
 
 namespace sllm {
@@ -125,6 +125,47 @@ __device__ __forceinline__ float w_scale(const void* s, size_t e, int n, int k0,
   }
 }
 
+// The other half of a lane's pair (rows 8 lanes, or mirrored 8-lane groups).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)dpp_u32<CTRL>((uint32_t)(u >> 32), 0u) << 32) |
+                                        dpp_u32<CTRL>((uint32_t)u, 0u));
+}
+
+// Sums of 16 values over the wave; lane l gets value l / 4's. Added in 64
+// bits, which takes six rounded additions out of every dot (a third of the
+// error), and with half the values given away at each of the first four steps
+// (17 additions instead of 96).
+__device__ __forceinline__ float wave_sum16(const float (&p)[16], int lane) {
+  double d[8], f[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {  // lanes 32 apart: upper half takes p[i + 8]
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[i]),
+                                                    __float_as_uint(p[i + 8]), false, false);
+    d[i] = (double)__uint_as_float(s[0]) + (double)__uint_as_float(s[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // rows 16 apart: odd rows take d[i + 4]
+    const uint64_t a = __builtin_bit_cast(uint64_t, d[i]);
+    const uint64_t b = __builtin_bit_cast(uint64_t, d[i + 4]);
+    const auto l = __builtin_amdgcn_permlane16_swap((uint32_t)a, (uint32_t)b, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(a >> 32), (uint32_t)(b >> 32),
+                                                    false, false);
+    f[i] = __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) +
+           __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+  }
+  double g[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)  // 8 apart (row_ror:8): bit 3 takes f[i + 2]
+    g[i] = (lane & 8 ? f[i + 2] : f[i]) + dpp_f64<0x128>(lane & 8 ? f[i] : f[i + 2]);
+  // mirrored within 8 lanes: bit 2 takes g[1]; then the four lanes' sums
+  double t = (lane & 4 ? g[1] : g[0]) + dpp_f64<0x141>(lane & 4 ? g[0] : g[1]);
+  t += dpp_f64<0xB1>(t);
+  t += dpp_f64<0x4E>(t);
+  return (float)t;
+}
+
 // SWIGLU = 1: rows (gate n, gate n+1, up n, up n+1) per wave, output h.
 // SWIGLU = 0: rows n..n+3 per wave of one weight, output y * row weight.
 template <int WF, typename TA, int SWIGLU>
@@ -137,6 +178,7 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(
     const void* __restrict__ s1, int N, int K,
     const float* __restrict__ row_w, float limit, float* __restrict__ out) {
   constexpr int KPC = ChunkK<WF>::value;  // K values per 16-byte chunk
+  constexpr int CH = KPC > 16 ? KPC / 2 : KPC;  // of them in a chain of sums
   int e, row_begin, rows;
   if (tile_info) {
     const int tile = blockIdx.y;
@@ -182,11 +224,9 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(
       const int ai = (gather_tokens && sorted_idx) ? sorted_idx[pos] / topk : pos;
       arow[r] = act + (size_t)ai * K;
     }
-    float part[4][4];
+    float part[16];  // weight row i, activation row r at 4 i + r
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) part[i][r] = 0.f;
+    for (int i = 0; i < 16; ++i) part[i] = 0.f;
     for (int c = lane; c < nch; c += 64) {
       const int k0 = c * KPC;
       float wv[4][KPC];
@@ -201,39 +241,31 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(
           load_act<TA, KPC>(arow[r] + k0, a);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            float d = 0.f;
+            float d[2] = {0.f, 0.f};
 #pragma unroll
-            for (int q = 0; q < KPC; ++q) d = fmaf(a[q], wv[i][q], d);
-            part[i][r] += d;
+            for (int q = 0; q < KPC; ++q)
+              d[q / CH] = fmaf(a[q], wv[i][q], d[q / CH]);
+            part[4 * i + r] += KPC > CH ? d[0] + d[1] : d[0];
           }
         }
       }
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) part[i][r] = wave_sum(part[i][r]);
-    // every lane holds the reduced sums; lane q*4+r writes output (q, r)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (lane == q * 4 + r && r < nr && (!SWIGLU || q < 2)) {
-          const int pos = row_begin + r0 + r;
-          if (SWIGLU) {
-            float g = part[q][r], u = part[q + 2][r];
-            if (limit > 0.f) {
-              u = fminf(fmaxf(u, -limit), limit);
-              g = fminf(g, limit);
-            }
-            out[(size_t)pos * N + nrow[q]] = silu_f32(g) * u;
-          } else {
-            float w = 1.f;
-            if (row_w) w = row_w[sorted_idx ? sorted_idx[pos] : pos];
-            out[(size_t)pos * N + nrow[q]] = part[q][r] * w;
-          }
-        }
+    // lane 16 q + 4 r writes output (q, r)
+    const float v = wave_sum16(part, lane);
+    const int q = lane >> 4, r = (lane >> 2) & 3;
+    const int pos = row_begin + r0 + r;
+    if (SWIGLU) {
+      float g = v, u = __shfl_xor(v, 32);
+      if (limit > 0.f) {
+        u = fminf(fmaxf(u, -limit), limit);
+        g = fminf(g, limit);
       }
+      if (lane % 4 == 0 && q < 2 && r < nr)
+        out[(size_t)pos * N + blockIdx.x * 8 + wave * 2 + q] = silu_f32(g) * u;
+    } else if (lane % 4 == 0 && r < nr) {
+      float w = 1.f;
+      if (row_w) w = row_w[sorted_idx ? sorted_idx[pos] : pos];
+      out[(size_t)pos * N + blockIdx.x * 16 + wave * 4 + q] = v * w;
     }
   }
 }
