@@ -136,6 +136,8 @@ SIGNATURES = {
     "sllm_moe_stream_dec_grid": (c_long, [c_long, c_int, c_long]),
     "sllm_moe_plan_query": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int,
                                     c_int, c_int, c_int, c_void_p, c_int]),
+    "sllm_moe_bf16_plan_query": (c_int, [c_int, c_int, c_int, c_int, c_int,
+                                         c_int, c_int, POINTER(c_int)]),
     "sllm_quantize_weight_fp8": (c_int, [P, c_int, c_int, c_int, P, P, P]),
     "sllm_quantize_weight_mxfp4": (c_int, [P, c_int, c_int, P, P, P]),
     "sllm_moe_qwen_workspace_bytes": (c_long, [POINTER(QwenArgs)]),

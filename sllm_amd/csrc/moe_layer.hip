@@ -33,7 +33,7 @@ struct Plan {
   int N;          // T * topk
   int bm, max_tiles;
   int bm_sh;  // decode: rows per tile of the shared expert's launches
-  int wide;   // bf16 weights: the tile of launch_wide
+  int wide;   // bf16 weights: the tile of launch_wide, 0 the GEMV
   // decode: K chunks of the streamed gate/up and down launches (routed /
   // shared) and partial-logit slices of the router GEMM
   int ks_up, ks_up_sh, ks_dn, ks_dn_sh, ks_r;
@@ -89,6 +89,10 @@ static int bf16_tile(long N, long E, long T, long I, bool has_shared) {
   return r >= 24 && tiles * (I / 128) >= device_cus() / 2 ? 4 : 3;
 }
 
+// bf16 weights, or not; the matrix-core kernel's loads need them 16-byte
+// aligned (wide_weights), the GEMV's do not.
+enum Bf16Weights { BF16_NONE, BF16_GEMV, BF16_WIDE };
+
 static size_t take(size_t& cur, size_t bytes) {
   size_t at = cur;
   cur += align_up(bytes ? bytes : 1, 256);
@@ -105,29 +109,31 @@ static bool pick_decode(int mode, int T) {
 // segment of the routed ones, and which routes every batch with the
 // multi-workgroup kernels.
 static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
-                      bool has_shared, bool need_logits, bool force_gemv,
+                      bool has_shared, bool need_logits, Bf16Weights bf16,
                       bool deepseek = false) {
   Plan p{};
   p.ks_up = p.ks_up_sh = p.ks_dn = p.ks_dn_sh = 1;
-  p.decode = force_gemv || pick_decode(mode, T);
+  p.decode = bf16 != BF16_NONE || pick_decode(mode, T);
   // The Qwen layer routes decode batches that fit one workgroup in one
   // fused launch (route_permute_small_fits), which would read every logit
   // slice through one CU: its router stays unsplit there. Up to
   // RI_MAX_ROUTE_T tokens the streamed layer routes inside the gate/up
   // launch instead, whose workgroups each read the slices: split there.
-  const bool inl_route = !deepseek && p.decode && !force_gemv &&
+  const bool inl_route = !deepseek && p.decode && bf16 == BF16_NONE &&
                          T <= RI_MAX_ROUTE_T && route_inline_fits(T, E, topk, 0) &&
                          route_inline_on();
   const bool fused_route = !deepseek && p.decode && !inl_route &&
                            route_permute_small_fits(T, E, topk);
   p.ks_r = p.decode && need_logits && !fused_route ? router_ksplit(T, H) : 1;
   p.N = T * topk;
+  int max_tiles = 0;
   if (p.decode) {
     // 16-row tiles (a touched expert's rows, mostly one tile), or 32 when
     // the experts average more than 16 rows (a dense MLP at 17-64 tokens),
     // so that each weight block is streamed once per 32 rows, not per 16
     p.bm = p.N > 16 * std::min(E, p.N) ? 32 : 16;
-    if (force_gemv) {  // bf16 weights: the matrix-core tiles (gemm_wide.hip)
+    max_tiles = (int)tile_bound(p.N, E, p.bm);
+    if (bf16 == BF16_WIDE) {  // the matrix-core tiles (gemm_wide.hip)
       p.wide = bf16_tile(p.N, E, T, I, has_shared);
       p.bm = p.wide == 1 ? 16 : (p.wide < 4 ? 32 : 64);
     }
@@ -145,7 +151,9 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
   p.sorted = take(c, (size_t)p.N * 4);
   p.rws = p.decode ? take(c, (size_t)p.N * 4) : 0;
   p.inv = take(c, (size_t)p.N * 4);
-  p.tiles = take(c, (size_t)p.max_tiles * 16);
+  // (bf16 weights: the GEMV's bound covers both kernels, as the size is asked
+  // for without the weights, whose alignment picks one)
+  p.tiles = take(c, (size_t)std::max(p.max_tiles, max_tiles) * 16);
   p.ntiles = take(c, 4);
   p.pscr = take(c, permute_scratch_bytes(p.N, E));
   // shared-expert gate, then (split router) its ks_r partial slices
@@ -154,7 +162,7 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
   if (!deepseek && !p.decode && need_logits && router_topk_fits(T, E, topk, H))
     p.rpart = take(c, router_part_bytes(T, E, topk));
   if (p.decode) {
-    if (!force_gemv) {  // the streamed kernels (the GEMV path does not split)
+    if (bf16 == BF16_NONE) {  // the streamed kernels (the others do not split)
       const long rt = p.max_tiles;
       const long sh_rt = has_shared ? (T + p.bm_sh - 1) / p.bm_sh : 0;
       // DeepSeek: MXFP4 routed and FP8 shared segments share a launch (a
@@ -271,7 +279,7 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
                   ? take(c, (size_t)2 * p.ks_up_sh * T * Is * 4) : 0;
     // (DeepSeek: the launches that route the batch in the gate/up launch,
     // whose router launch clears the counters)
-    if (!force_gemv &&
+    if (bf16 == BF16_NONE &&
         (deepseek ? T <= RI_MAX_ROUTE_T : (T <= DEC_FUSE_MAX_T || p.sk_up))) {
       p.fcnt_on = true;
       p.fcnt = take(c, (size_t)(dec_fuse_counters(p.N, T, I, has_shared ? Is : 0) +
@@ -405,7 +413,8 @@ long sllm_moe_qwen_workspace_bytes(const sllm_moe_qwen_args* a) {
   }
   const bool sh = a->su != nullptr;
   return (long)make_plan(a->T, a->H, a->E, a->I, sh ? a->Is : 0, a->topk,
-                         a->mode, sh, !a->logits_given, a->wdtype == 1)
+                         a->mode, sh, !a->logits_given,
+                         a->wdtype == 1 ? BF16_WIDE : BF16_NONE)
       .total;
 }
 
@@ -439,7 +448,9 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
   const int Is = sh ? a->Is : 0;
   const int wf = bf16w ? 2 : 0;  // gemv weight format
   const Plan p = make_plan(T, H, E, I, Is, k, a->mode, sh, !a->logits_given,
-                           bf16w);
+                           !bf16w             ? BF16_NONE
+                           : wide_weights(a) ? BF16_WIDE
+                                             : BF16_GEMV);
   SLLM_REQUIRE(ws_bytes >= (long)p.total,
                "sllm_moe_qwen_forward: workspace %ld < %zu bytes", ws_bytes,
                p.total);
@@ -725,7 +736,7 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
                                             y_sh, T, H, a->out_f32, a->out,
                                             p.ks_dn, (long)p.N * H, p.ks_dn_sh,
                                             (long)T * H, st));
-    } else if (bf16w && wide_weights(a)) {
+    } else if (p.wide) {
       // bf16 weights on the matrix cores, routed and shared segments in one
       // launch per projection
       float* h_sh = sh ? (float*)(ws + p.hq_sh) : nullptr;
@@ -1027,7 +1038,7 @@ long sllm_moe_ds_workspace_bytes(const sllm_moe_ds_args* a) {
   }
   const bool sh = a->s1 != nullptr;
   return (long)make_plan(a->T, a->H, a->E, a->I, sh ? a->Is : 0, a->topk,
-                         a->mode, sh, !a->logits_given, false, true)
+                         a->mode, sh, !a->logits_given, BF16_NONE, true)
       .total;
 }
 
@@ -1044,7 +1055,7 @@ int sllm_moe_plan_query(int deepseek, int T, int H, int E, int I, int Is,
                "sllm_moe_plan_query: bad args (T=%d H=%d E=%d I=%d Is=%d "
                "k=%d mode %d, %d outputs)", T, H, E, I, Is, topk, mode, n_out);
   const Plan p = make_plan(T, H, E, I, Is, topk, mode, Is > 0, !logits_given,
-                           false, deepseek != 0);
+                           BF16_NONE, deepseek != 0);
   for (int i = 0; i < SLLM_MOE_PLAN_FIELDS; ++i) out[i] = 0;
   out[0] = p.decode;
   out[1] = p.bm;
@@ -1087,6 +1098,21 @@ int sllm_moe_plan_query(int deepseek, int T, int H, int E, int I, int Is,
     out[11 + 3 * j] = cb;
     out[12 + 3 * j] = dec_launch_grid(items[j], cb);
   }
+  return 0;
+}
+
+// Host plan query of the bf16-weight Qwen layer (no device work).
+int sllm_moe_bf16_plan_query(int T, int H, int E, int I, int Is, int topk,
+                             int aligned, int* out) {
+  SLLM_REQUIRE(out && T > 0 && H > 0 && E > 0 && I > 0 && Is >= 0 && topk > 0 &&
+                   topk <= E && H % 256 == 0 && I % 128 == 0 && Is % 128 == 0,
+               "sllm_moe_bf16_plan_query: bad args (T=%d H=%d E=%d I=%d Is=%d "
+               "k=%d)", T, H, E, I, Is, topk);
+  const Plan p = make_plan(T, H, E, I, Is, topk, SLLM_MOE_MODE_AUTO, Is > 0, true,
+                           aligned ? BF16_WIDE : BF16_GEMV);
+  out[0] = p.wide;
+  out[1] = p.bm;
+  out[2] = p.max_tiles;
   return 0;
 }
 
@@ -1173,7 +1199,7 @@ int sllm_moe_ds_forward(const sllm_moe_ds_args* a) {
   const float L = a->swiglu_limit;
   const bool dense = dense_layer(a);
   const Plan p = make_plan(T, H, E, I, Is, k, a->mode, sh, !a->logits_given,
-                           false, true);
+                           BF16_NONE, true);
   SLLM_REQUIRE(a->workspace_bytes >= (long)p.total,
                "sllm_moe_ds_forward: workspace %ld < %zu bytes",
                a->workspace_bytes, p.total);

@@ -205,6 +205,85 @@ def test_bf16_layer_tiles(T, k, shared, H):
     assert rel < 2e-6, rel
 
 
+def _off(a, by=8):
+    """A device copy of `a` that begins `by` bytes past an aligned address."""
+    from sllm_amd.runtime import to_device_raw
+    raw = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    buf = to_device_raw(np.concatenate([np.zeros(by, np.uint8), raw]))
+    return buf, buf.ptr + by
+
+
+# rows an expert below and above 16, below and above a 64-row tile
+@pytest.mark.parametrize("T,k,shared", [(3, 2, True), (40, 2, False), (90, 2, True), (300, 3, True)])
+def test_bf16_layer_unaligned_weights(T, k, shared):
+    """Weights 8 bytes past a 16-byte boundary: the GEMV, against the
+    per-token loop."""
+    import ctypes
+    from sllm_amd import _lib
+    from sllm_amd.moe import qwen_workspace_bytes
+    from sllm_amd.runtime import DeviceBuffer, sync, to_bf16, to_device_raw
+    rng = np.random.default_rng(T)
+    H, E, I = 256, 5, 128
+
+    def w(*shape):
+        return bf((rng.standard_normal(shape) * 0.05).astype(np.float32))
+    x = bf(rng.standard_normal((T, H)).astype(np.float32))
+    W = dict(router_w=w(E, H), wg=w(E, I, H), wu=w(E, I, H), wd=w(E, H, I))
+    if shared:
+        W.update(sg=w(I, H), su=w(I, H), sd=w(H, I), sgl=w(1, H))
+    logits = DeviceBuffer(T * E * 4)
+    out = DeviceBuffer(T * H * 4)
+    nb = qwen_workspace_bytes(T, H, E, I, I if shared else 0, k, has_shared=shared, wdtype=1)
+    ws, xb = DeviceBuffer(nb), to_device_raw(to_bf16(x))
+    a = _lib.QwenArgs()
+    a.T, a.H, a.E, a.I, a.Is, a.topk = T, H, E, I, I if shared else 0, k
+    a.out_f32, a.wdtype, a.renorm_eps = 1, 1, 1e-20
+    a.x, a.out, a.logits_out, a.workspace, a.workspace_bytes = xb.ptr, out.ptr, logits.ptr, ws.ptr, nb
+    keep = {}
+    for name, v in W.items():
+        buf, p = _off(to_bf16(v), 0 if name in ("router_w", "sgl") else 8)
+        keep[name] = buf
+        setattr(a, name, p)
+    _lib.check(_lib.lib().sllm_moe_qwen_forward(ctypes.byref(a)), "qwen")
+    sync()
+    want = qm.moe_block_grouped(x, logits.copy_host().reshape(T, E), W["wg"], W["wu"], W["wd"], k,
+                                (W["sg"], W["su"], W["sd"], W["sgl"]) if shared else None)
+    got = out.copy_host().reshape(T, H)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 2e-6
+
+
+@pytest.mark.parametrize("M", [2, 40, 70])
+def test_unaligned_linears(M):
+    """FP8 and MXFP4 weights 8 bytes past a 16-byte boundary, and FP8
+    activations 4 past: the GEMV up to 64 rows, the tiled kernel above."""
+    from sllm_amd import deepseek, fp8
+    from sllm_amd.runtime import DeviceBuffer, sync
+    rng = np.random.default_rng(M)
+    N, K = 128, 256
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    q = rng.integers(0, 0x70, (N, K), dtype=np.uint8)
+    s = (rng.random((1, 2)) + 0.5).astype(np.float32)
+    p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    sc = rng.integers(115, 130, (N, K // 32), dtype=np.uint8)
+    out = DeviceBuffer(M * N * 4)
+    bufs = [_off(a, 0), _off(q), _off(s, 0), _off(a, 4), _off(p), _off(sc, 0)]
+    d = [b[1] for b in bufs]
+
+    def check(wd):
+        sync()
+        got = out.copy_host().reshape(M, N)
+        # the tiled kernel adds K products one by one: (K + 2) 2^-24
+        mag = np.abs(a).astype(np.float64) @ np.abs(wd).astype(np.float64).T
+        err = np.abs(got - a.astype(np.float64) @ wd.astype(np.float64).T)
+        assert np.all(err <= (K + 2) * 2.0 ** -24 * mag)
+    fp8.fp8_gemm_dev(d[0], d[1], d[2], out, M, N, K)
+    check(codecs.dequant_fp8_block(q, s))
+    fp8.fp8_gemm_dev(d[3], d[1], d[2], out, M, N, K)
+    check(codecs.dequant_fp8_block(q, s))
+    deepseek.fp4_moe_linear_dev(d[0], d[4], d[5], out, M, N, K)
+    check(codecs.dequant_fp4_block(p, sc))
+
+
 @pytest.mark.parametrize("T", [3, 40])
 def test_bf16_layer_infinity(T):
     """An infinite activation under positive weights leaves its token
