@@ -157,8 +157,11 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
   p.ntiles = take(c, 4);
   p.pscr = take(c, permute_scratch_bytes(p.N, E));
   // shared-expert gate, then (split router) its ks_r partial slices
-  const int ks_g = p.decode && T > DECODE_MAX_T ? router_one_round(H) : p.ks_r;
-  p.gate = take(c, (size_t)(ks_g > 1 ? 1 + ks_g : 1) * T * 4);
+  // (a short prompt's slices: in the logits' place, see below, or with fewer
+  // experts than slices here)
+  const int ks_g = p.decode && need_logits && router_short(T, E) ? router_one_round(H) : p.ks_r;
+  const bool gate_far = ks_g > p.ks_r && E > ks_g;
+  p.gate = take(c, (size_t)(ks_g > 1 && !gate_far ? 1 + ks_g : 1) * T * 4);
   if (!deepseek && !p.decode && need_logits && router_topk_fits(T, E, topk, H))
     p.rpart = take(c, router_part_bytes(T, E, topk));
   if (p.decode) {
@@ -298,7 +301,8 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
     p.y_sh = has_shared ? take(c, (size_t)T * H * 2) : 0;
   }
   // A short prompt's router slices lie in the y rows, which the down launch
-  // writes after the routing launch has read them.
+  // writes after the routing launch has read them; so the logits' own place is
+  // free for the gate's, and the call needs no more workspace than unsplit.
   p.ks_l = p.ks_r;
   if (need_logits && router_short(T, E)) {
     const size_t yb = p.decode ? (size_t)p.ks_dn * p.N * H * 4 : (size_t)p.N * H * 2;
@@ -306,6 +310,7 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
     if (ks > 1 && (size_t)ks * T * E * 4 <= yb) {
       p.rlog = p.y;
       p.ks_l = ks;
+      if (gate_far) p.gate = p.logits;  // (T E floats, of which 1 + ks slices)
     }
   }
   p.total = c;

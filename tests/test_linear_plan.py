@@ -26,6 +26,31 @@ def test_unaligned_bf16_layer_keeps_the_gemvs_tiles(T, H, E, I, Is, k):
     assert bound == _lib.lib().sllm_moe_tile_bound(T * k, E, bm)
 
 
+def _workspace(T, H, E, I, Is, k, logits_given):
+    a = _lib.QwenArgs()
+    a.T, a.H, a.E, a.I, a.Is, a.topk, a.wdtype = T, H, E, I, Is, k, 1
+    a.su = 8 if Is else None
+    a.logits_given = logits_given
+    return _lib.lib().sllm_moe_qwen_workspace_bytes(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("T", [65, 130, 1000, 4000])
+@pytest.mark.parametrize("logits_given", [0, 1])
+@pytest.mark.parametrize("H,E,I,Is,k", [(1024, 16, 512, 512, 4), (2048, 32, 768, 0, 4),
+                                        (7168, 256, 2048, 2048, 8), (2048, 512, 512, 512, 10)])
+def test_bf16_workspace_holds_no_router_slices(T, H, E, I, Is, k, logits_given):
+    """Above 64 tokens the workspace is that of the unsplit router (a call at
+    the limit of the fixed scratch stays within it): routing tables, h, y."""
+    N, al = T * k, lambda b: -(-b // 256) * 256
+    bm = 32 if N > 16 * min(E, N) else 16
+    tables = [T * E * 4 * (1 - logits_given), N * 4, N * 4, E * 4, (E + 1) * 4, N * 4, N * 4,
+              N * 4, _lib.lib().sllm_moe_tile_bound(N, E, bm) * 16, 4,
+              al(-(-N // 1024) * E * 4), T * 4, N * I * 4, N * H * 4]
+    if Is:
+        tables += [T * Is * 4, T * H * 4]
+    assert _workspace(T, H, E, I, Is, k, logits_given) == sum(al(b) for b in tables)
+
+
 def test_bf16_plan_rejects_bad_sizes():
     out = (ctypes.c_int * 4)()
     assert _lib.lib().sllm_moe_bf16_plan_query(4, 100, 8, 128, 0, 2, 1, out) == -1
