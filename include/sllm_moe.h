@@ -258,7 +258,9 @@ int sllm_moe_plan_query(int deepseek, int T, int H, int E, int I, int Is,
 /* The same for the Qwen layer with bf16 weights (wdtype 1; aligned: x and
  * the weights on 16 bytes): out[0] the routed experts' kernel (0: the GEMV,
  * 1-4: the matrix-core kernel's tile, of 16 x 32, 32 x 64, 32 x 128 or
- * 64 x 256 rows x columns), out[1] rows per tile, out[2] their bound. */
+ * 64 x 256 rows x columns), out[1] rows per tile, out[2] their bound,
+ * out[3] the shared expert's kernel where the routed ones take the GEMV (it
+ * shares the matrix-core kernel's launches otherwise). */
 int sllm_moe_bf16_plan_query(int T, int H, int E, int I, int Is, int topk,
                              int aligned, int* out);
 /* Synthetic-weight quantizers (data preparation): FP8 128x128 block

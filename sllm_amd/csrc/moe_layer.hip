@@ -33,7 +33,8 @@ struct Plan {
   int N;          // T * topk
   int bm, max_tiles;
   int bm_sh;  // decode: rows per tile of the shared expert's launches
-  int wide;   // bf16 weights: the tile of launch_wide, 0 the GEMV
+  int wide;     // bf16 weights: the tile of launch_wide, 0 the GEMV
+  int wide_sh;  // the shared expert's, where it has launches of its own
   // decode: K chunks of the streamed gate/up and down launches (routed /
   // shared) and partial-logit slices of the router GEMM
   int ks_up, ks_up_sh, ks_dn, ks_dn_sh, ks_r;
@@ -89,6 +90,26 @@ static int bf16_tile(long N, long E, long T, long I, bool has_shared) {
   return r >= 24 && tiles * (I / 128) >= device_cus() / 2 ? 4 : 3;
 }
 
+// Whether the bf16 layer's routed experts run on the GEMV: with few rows a
+// touched expert (E (1 - (1 - 1/E)^N) of them), where it streams the weights
+// faster: below three, or with several experts, most of which then have no
+// more than the four rows of one pass, below an average of 3.4. GEMV / matrix
+// cores, us: H 2048 E 32 I 768 top-4, 3 / 16 / 24 / 40 tokens (1.2 / 2.3 / 3.2 /
+// 5 rows) 36 / 57, 71 / 84, 85 / 87, 107 / 103; E 128 top-8, 8 / 48 / 64 tokens
+// (1.3 / 3.2 / 4.1) 107 / 142, 258 / 272, 310 / 284; E 1 I 5632, 1 / 2 / 4
+// tokens 33 / 47, 39 / 47, 48 / 47. A shared
+// expert then has launches of its own, 8 us or more, which the touched weights
+// repay from 64 MB at one or two tokens (E 128 top-8 with a shared expert, 1
+// token, 73 MB: 42 / 50), from 150 MB above (E 512 I 512 top-10, 8 / 64 tokens
+// 133 / 156, 463 / 631; E 32, 6 tokens, 161 MB 62 / 76) and below 2.25 rows (20
+// tokens, 2.7 rows 121 / 103). Short of that: E 16 I 512 top-4 at 8 tokens 43 /
+// 36, E 64 I 256 top-6 at 16 (78 MB) 56 / 42.
+static bool bf16_gemv(long N, long E, long T, long I, long H, bool has_shared) {
+  const double touched = E * (1.0 - std::pow(1.0 - 1.0 / E, (double)N));
+  if (!has_shared) return N < (E > 1 ? 3.4 : 3.0) * touched;
+  return N < 2.25 * touched && touched * 6 * H * I >= (T < 3 ? 64e6 : 150e6);
+}
+
 // bf16 weights, or not; the matrix-core kernel's loads need them 16-byte
 // aligned (wide_weights), the GEMV's do not.
 enum Bf16Weights { BF16_NONE, BF16_GEMV, BF16_WIDE };
@@ -133,7 +154,10 @@ static Plan make_plan(int T, int H, int E, int I, int Is, int topk, int mode,
     // so that each weight block is streamed once per 32 rows, not per 16
     p.bm = p.N > 16 * std::min(E, p.N) ? 32 : 16;
     max_tiles = (int)tile_bound(p.N, E, p.bm);
-    if (bf16 == BF16_WIDE) {  // the matrix-core tiles (gemm_wide.hip)
+    if (bf16 == BF16_WIDE && bf16_gemv(p.N, E, T, I, H, has_shared)) {
+      // the shared expert, with all T rows, by the same line
+      p.wide_sh = has_shared && T >= 3 ? bf16_tile(T, 1, T, Is, false) : 0;
+    } else if (bf16 == BF16_WIDE) {  // the matrix-core tiles (gemm_wide.hip)
       p.wide = bf16_tile(p.N, E, T, I, has_shared);
       p.bm = p.wide == 1 ? 16 : (p.wide < 4 ? 32 : 64);
     }
@@ -741,9 +765,10 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
                                             y_sh, T, H, a->out_f32, a->out,
                                             p.ks_dn, (long)p.N * H, p.ks_dn_sh,
                                             (long)T * H, st));
-    } else if (p.wide) {
-      // bf16 weights on the matrix cores, routed and shared segments in one
-      // launch per projection
+    } else {
+      // unpacked weights: bf16 on the matrix cores, routed and shared segments
+      // in one launch per projection, or a launch each with the GEMV (FP8
+      // always; bf16_gemv's batches, the shared segment by its own rows)
       float* h_sh = sh ? (float*)(ws + p.hq_sh) : nullptr;
       y_sh = sh ? (float*)(ws + p.y_sh) : nullptr;
       WideSeg r1{}, s1{};
@@ -755,7 +780,11 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
       s1.w0 = (const uint8_t*)a->sg; s1.w1 = (const uint8_t*)a->su;
       s1.N = Is; s1.K = H; s1.out = h_sh;
       STAGE(clk, SLLM_MOE_STAGE_EXPERT_UP,
-            launch_wide(WD_BF16, 1, p.wide, r1, sh ? &s1 : nullptr, k, st));
+            p.wide ? launch_wide(WD_BF16, 1, p.wide, r1, sh ? &s1 : nullptr, k, st)
+                   : launch_gemv(wf, 1, a->x, 1, 1, sorted, k, p.N, tiles, ntiles,
+                                 p.max_tiles, offsets, (const uint8_t*)a->wg,
+                                 a->wg_s, (const uint8_t*)a->wu, a->wu_s, I, H,
+                                 nullptr, 0.f, h, st));
       WideSeg r2{}, s2{};
       r2.a = h; r2.sorted_idx = sorted;
       r2.tile_info = tiles; r2.num_tiles = ntiles; r2.max_tiles = p.max_tiles;
@@ -764,33 +793,26 @@ static int qwen_forward_ws(const sllm_moe_qwen_args* a, char* ws,
       s2.w0 = (const uint8_t*)a->sd; s2.N = H; s2.K = Is; s2.row_w = gate;
       s2.out = y_sh;
       STAGE(clk, SLLM_MOE_STAGE_EXPERT_DOWN,
-            launch_wide(WD_BF16, 0, p.wide, r2, sh ? &s2 : nullptr, k, st));
+            p.wide ? launch_wide(WD_BF16, 0, p.wide, r2, sh ? &s2 : nullptr, k, st)
+                   : launch_gemv(wf, 0, h, 0, 0, sorted, k, p.N, tiles, ntiles,
+                                 p.max_tiles, offsets, (const uint8_t*)a->wd,
+                                 a->wd_s, nullptr, nullptr, H, I, w, 0.f, y, st));
+      if (sh && !p.wide) {
+        STAGE(clk, SLLM_MOE_STAGE_SHARED_UP,
+              p.wide_sh ? launch_wide(WD_BF16, 1, p.wide_sh, s1, nullptr, 1, st)
+                        : launch_gemv(wf, 1, a->x, 1, 0, nullptr, k, T, nullptr,
+                                      nullptr, 1, nullptr, (const uint8_t*)a->sg,
+                                      a->sg_s, (const uint8_t*)a->su, a->su_s, Is,
+                                      H, nullptr, 0.f, h_sh, st));
+        STAGE(clk, SLLM_MOE_STAGE_SHARED_DOWN,
+              p.wide_sh ? launch_wide(WD_BF16, 0, p.wide_sh, s2, nullptr, 1, st)
+                        : launch_gemv(wf, 0, h_sh, 0, 0, nullptr, k, T, nullptr,
+                                      nullptr, 1, nullptr, (const uint8_t*)a->sd,
+                                      a->sd_s, nullptr, nullptr, H, Is, gate, 0.f,
+                                      y_sh, st));
+      }
       STAGE(clk, SLLM_MOE_STAGE_COMBINE,
             launch_combine(y, 1, inv, k, y_sh, T, H, a->out_f32, a->out, st));
-    } else {
-    STAGE(clk, SLLM_MOE_STAGE_EXPERT_UP,
-          launch_gemv(wf, 1, a->x, 1, 1, sorted, k, p.N, tiles, ntiles,
-          p.max_tiles, offsets, (const uint8_t*)a->wg, a->wg_s,
-          (const uint8_t*)a->wu, a->wu_s, I, H, nullptr, 0.f, h, st));
-    STAGE(clk, SLLM_MOE_STAGE_EXPERT_DOWN,
-          launch_gemv(wf, 0, h, 0, 0, sorted, k, p.N, tiles, ntiles, p.max_tiles,
-          offsets, (const uint8_t*)a->wd, a->wd_s, nullptr, nullptr,
-          H, I, w, 0.f, y, st));
-    if (sh) {
-      float* h_sh = (float*)(ws + p.hq_sh);
-      y_sh = (float*)(ws + p.y_sh);
-      STAGE(clk, SLLM_MOE_STAGE_SHARED_UP,
-            launch_gemv(wf, 1, a->x, 1, 0, nullptr, k, T, nullptr, nullptr, 1,
-            nullptr, (const uint8_t*)a->sg, a->sg_s,
-            (const uint8_t*)a->su, a->su_s, Is, H, nullptr, 0.f,
-            h_sh, st));
-      STAGE(clk, SLLM_MOE_STAGE_SHARED_DOWN,
-            launch_gemv(wf, 0, h_sh, 0, 0, nullptr, k, T, nullptr, nullptr, 1,
-            nullptr, (const uint8_t*)a->sd, a->sd_s, nullptr,
-            nullptr, H, Is, gate, 0.f, y_sh, st));
-    }
-    STAGE(clk, SLLM_MOE_STAGE_COMBINE,
-          launch_combine(y, 1, inv, k, y_sh, T, H, a->out_f32, a->out, st));
     }
   } else {
     uint8_t* xq = (uint8_t*)(ws + p.xq);
@@ -1118,6 +1140,7 @@ int sllm_moe_bf16_plan_query(int T, int H, int E, int I, int Is, int topk,
   out[0] = p.wide;
   out[1] = p.bm;
   out[2] = p.max_tiles;
+  out[3] = p.wide_sh;
   return 0;
 }
 

@@ -205,6 +205,33 @@ def test_bf16_layer_tiles(T, k, shared, H):
     assert rel < 2e-6, rel
 
 
+# with a shared expert on the GEMV (1, 2 tokens), the 16-row tiles and the
+# 32-row ones; above 64 tokens (the router's launch split); without a shared
+# expert
+@pytest.mark.parametrize("T,E,k,shared,H,I", [
+    (1, 24, 4, True, 2048, 1408), (2, 24, 4, True, 2048, 1408), (3, 24, 4, True, 2048, 1408),
+    (10, 24, 4, True, 2048, 1408), (20, 64, 5, True, 1280, 512), (70, 80, 2, True, 2048, 256),
+    (7, 16, 2, False, 256, 128), (80, 64, 2, False, 1280, 128),
+    (2, 1, 1, False, 512, 256)])
+def test_bf16_layer_few_rows(T, E, k, shared, H, I):
+    """Few rows an expert: the routed GEMV with each kernel of the shared
+    expert, against the per-token loop."""
+    from sllm_amd.moe import QwenMoE
+    rng = np.random.default_rng(T + E)
+    Is = 384
+
+    def w(*shape):
+        return bf(rng.standard_normal(shape, dtype=np.float32) * np.float32(0.05))
+    x = bf(rng.standard_normal((T, H)).astype(np.float32))
+    rw, wg, wu, wd = w(E, H), w(E, I, H), w(E, I, H), w(E, H, I)
+    sg, su, sd, sgl = (w(Is, H), w(Is, H), w(H, Is), w(1, H)) if shared else (None,) * 4
+    layer = QwenMoE(rw, wg, wu, wd, sg=sg, su=su, sd=sd, sgl=sgl, top_k=k)
+    got, r = layer.forward(x, return_routing=True)
+    want = qm.moe_block_grouped(x, r["logits"], wg, wu, wd, k,
+                                (sg, su, sd, sgl) if shared else None)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 2e-6
+
+
 def _off(a, by=8):
     """A device copy of `a` that begins `by` bytes past an aligned address."""
     from sllm_amd.runtime import to_device_raw

@@ -26,6 +26,26 @@ def test_unaligned_bf16_layer_keeps_the_gemvs_tiles(T, H, E, I, Is, k):
     assert bound == _lib.lib().sllm_moe_tile_bound(T * k, E, bm)
 
 
+# tokens below / from the line in rows a touched expert
+@pytest.mark.parametrize("H,E,I,Is,k,below,above", [
+    (2048, 32, 768, 0, 4, (1, 3, 8, 24), (32, 64)), (2048, 128, 768, 0, 8, (1, 32, 48), (64,)),
+    (2048, 1, 5632, 0, 1, (1, 2), (3, 4)), (4096, 8, 14336, 0, 2, (1, 12), (16,)),
+    # a shared expert, whose launches of its own cost more beside few weights
+    (2048, 512, 512, 512, 10, (2, 3, 64), (1, 130)), (1024, 16, 512, 512, 4, (), (1, 8, 64)),
+    (2048, 32, 768, 768, 4, (2, 6, 12), (1, 5, 16, 24))])
+def test_bf16_layer_kernel_by_rows(H, E, I, Is, k, below, above):
+    """Few rows a touched expert run on the GEMV: below 3.4 (one expert 3,
+    beside a shared one 2.25 and enough weights)."""
+    for T in below:
+        tile, bm, bound, sh = _bf16_plan(T, H, E, I, Is, k)
+        assert tile == 0 and bm == (32 if T * k > 16 * min(E, T * k) else 16), T
+        assert bound == _lib.lib().sllm_moe_tile_bound(T * k, E, bm)
+        assert (sh > 0) == (Is > 0 and T >= 3), T
+    for T in above:
+        tile, bm, _, sh = _bf16_plan(T, H, E, I, Is, k)
+        assert tile > 0 and bm == {1: 16, 2: 32, 3: 32, 4: 64}[tile] and sh == 0, T
+
+
 def _workspace(T, H, E, I, Is, k, logits_given):
     a = _lib.QwenArgs()
     a.T, a.H, a.E, a.I, a.Is, a.topk, a.wdtype = T, H, E, I, Is, k, 1
