@@ -263,6 +263,13 @@ int sllm_moe_plan_query(int deepseek, int T, int H, int E, int I, int Is,
  * shares the matrix-core kernel's launches otherwise). */
 int sllm_moe_bf16_plan_query(int T, int H, int E, int I, int Is, int topk,
                              int aligned, int* out);
+/* The same for the FP8 (fp4 = 0) and MXFP4 (1; block_h unread) linears
+ * (aligned: activations, weight codes and result on 16 bytes): 0-4 the
+ * matrix-core kernel's tile (16 x 16, 16 x 32, 32 x 64, 32 x 128, then FP8
+ * 32 x 256 or MXFP4 64 x 128 rows x columns), 5 the GEMV, 6 the tiled
+ * kernel; -1 for bad sizes. */
+int sllm_linear_plan_query(int fp4, int M, int N, int K, int block_h,
+                           int block_w, int aligned);
 /* Synthetic-weight quantizers (data preparation): FP8 128x128 block
  * (s = amax/448, optionally its power-of-two ceiling) and MXFP4 per 32. */
 int sllm_quantize_weight_fp8(const float* w, int N, int K, int pow2,

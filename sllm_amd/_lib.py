@@ -138,6 +138,7 @@ SIGNATURES = {
                                     c_int, c_int, c_int, c_void_p, c_int]),
     "sllm_moe_bf16_plan_query": (c_int, [c_int, c_int, c_int, c_int, c_int,
                                          c_int, c_int, POINTER(c_int)]),
+    "sllm_linear_plan_query": (c_int, [c_int] * 7),
     "sllm_quantize_weight_fp8": (c_int, [P, c_int, c_int, c_int, P, P, P]),
     "sllm_quantize_weight_mxfp4": (c_int, [P, c_int, c_int, P, P, P]),
     "sllm_moe_qwen_workspace_bytes": (c_long, [POINTER(QwenArgs)]),

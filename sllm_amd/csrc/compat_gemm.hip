@@ -120,6 +120,67 @@ int launch_tiled_gemm(const void* a, int a_bf16, const BDesc& bd, float* c,
 using namespace sllm;
 
 namespace {
+
+// Where a quantized linear runs: a tile of the matrix-core kernel
+// (launch_wide's 0-4), the layer's unpacked-weight GEMV, or the tiled kernel.
+enum { LIN_GEMV = 5, LIN_TILED = 6 };
+
+// One row always streams through the GEMV (128 x 128 blocks). Two to four rows
+// do where it streams B faster than the matrix cores' tiles, which few rows
+// leave mostly empty. us, GEMV / matrix cores, repeated (weights from memory):
+// - up to 32 columns a CU (one round of the 16-row tiles) short K only: 2
+//   rows 2048 x 2048 4.3 / 5.8 (9 / 9), 4096 x 4096 7.0 / 7.9 (15 / 14), 2048
+//   x 7168 8.2 / 9.9 (19 / 16), 7168 x 7168 15.1 / 14.1 (30 / 26); 3 rows 7168
+//   x 2048 6.0 / 7.7 (13 / 12), 4096 x 4096 7.8 / 8.0 (18 / 14); 4 rows 9.9 / 8.0
+// - up to 48 (one round of three GEMV workgroups of 16 a CU, 32-row tiles
+//   there): 12288 x 4096, 2 / 4 / 5 rows 11.8 / 20.9 (26 / 29), 17.0 / 20.9 (32 /
+//   29), 23.9 / 20.9 (39 / 29)
+// - up to 64 (one round of 32 x 64 tiles, two of the GEMV): 14336 x 4096, 2
+//   rows 21.2 / 21.6 (34 / 29)
+// - above: 2 rows (17408 x 5120 24.3 / 38.9 (44 / 56), 64000 x 4096 62.1 / 60.1
+//   (104 / 130)), 3 up to 96 (18432 x 7168 41.8 / 50.8 (69 / 70), 32000 x 4096
+//   41.6 / 32.3 (63 / 67)); 4 rows 17408 x 5120 36.6 / 38.9 (56 / 56), 20480 x
+//   2048 18.2 / 17.4 (28 / 26).
+bool fp8_few_rows(int M, int N, int K, int cus) {
+  if (M == 1) return true;
+  if (K < 1024 || M > 4) return false;
+  if (N <= 32 * cus) return K <= (M == 2 ? 4096 : M == 3 ? 2048 : 0);
+  if (N <= 48 * cus) return true;
+  return N > 64 * cus && (M == 2 || (M == 3 && N <= 96 * cus));
+}
+
+// The same for MXFP4: 2 rows 4096 x 4096 7.9 / 10.3 (14 / 15), 2048 x 7168 12.5 /
+// 13.6 (22 / 19), 8192 x 4096 11.4 / 15.6 (19 / 20), 14336 x 4096 21.1 / 25.3
+// (32 / 31), 18432 x 7168 52.3 / 59.8 (70 / 68), 20480 x 2048 15.1 / 29.2 (27 /
+// 35), 32000 x 4096 43.8 / 40.2 (58 / 52), 256 x 256 6.2 / 4.3; 3 rows 2048 x 2048
+// 6.0 / 7.4 (10 / 11), 20480 x 2048 19.1 / 29.1 (32 / 35), 4096 x 4096 9.6 / 10.2
+// (16 / 15), 14336 x 4096 27.5 / 25.2 (39 / 31); 4 rows 7168 x 2048 10.4 / 10.7
+// (16 / 15), 20480 x 2048 23.2 / 29.2 (37 / 35).
+bool fp4_few_rows(int M, int N, int K, int cus) {
+  if (M == 1) return true;
+  if (K < 1024 || N > 96 * cus) return false;
+  if (M == 2) return K <= 4096 || N > 32 * cus;
+  return K <= 2048 && (M == 3 ? K > 1024 : M == 4 && N > 64 * cus);
+}
+
+// FP8: the matrix cores take scale blocks of 4 n rows by 64 2^m columns, the
+// GEMV the loader's 128 x 128. fits: wide_fits and no null pointer.
+int fp8_route(int M, int N, int K, int bh, int bw, bool fits) {
+  const int cus = device_cus();
+  const bool gemv = bh == 128 && bw == 128 && M <= 64 && N % 128 == 0 && K % 128 == 0;
+  const bool wide = M > 1 && fits && bh % 4 == 0 && bw % 64 == 0 && bw == 64 << __builtin_ctz(bw / 64);
+  if (gemv && (!wide || fp8_few_rows(M, N, K, cus))) return LIN_GEMV;
+  return wide ? wide_tile(WD_FP8, M, N, cus) : LIN_TILED;
+}
+
+int fp4_route(int M, int N, int K, int bw, bool fits) {
+  const int cus = device_cus();
+  const bool gemv = bw == 32 && M <= 64 && K % 32 == 0 && N % 16 == 0;
+  const bool wide = M > 1 && N > 0 && fits && bw == 32;
+  if (gemv && (!wide || fp4_few_rows(M, N, K, cus))) return LIN_GEMV;
+  return wide ? wide_tile(WD_FP4, M, N, cus) : LIN_TILED;
+}
+
 struct Tmp {
   void* p = nullptr;
   ~Tmp() {
@@ -130,29 +191,31 @@ struct Tmp {
 
 extern "C" {
 
+// Host query (no device work): which kernel the FP8 and MXFP4 linears take.
+int sllm_linear_plan_query(int fp4, int M, int N, int K, int block_h,
+                           int block_w, int aligned) {
+  SLLM_REQUIRE(M > 0 && N > 0 && K > 0 && block_h > 0 && block_w > 0,
+               "sllm_linear_plan_query: bad dims");
+  const bool fits = aligned && wide_fits(nullptr, nullptr, nullptr, K);
+  return fp4 ? fp4_route(M, N, K, block_w, fits) : fp8_route(M, N, K, block_h, block_w, fits);
+}
+
 int sllm_fp8_gemm_dev(const float* A, const unsigned char* B,
                       const float* scale_inv, float* C, int M, int N, int K,
                       int block_h, int block_w) {
   SLLM_REQUIRE(M > 0 && N > 0 && K > 0 && block_h > 0 && block_w > 0,
                "sllm_fp8_gemm: bad dims");
   SLLM_REQUIRE(scale_inv, "sllm_fp8_gemm: null scale");
-  // from two rows: the matrix cores (one row: the GEMV below streams B as
-  // fast with less to set up, 8.2 against 8.7 us at 4096 x 4096; two rows
-  // 10.0 against 8.7, 32 rows 76 against 13, 512 rows 738 against 55 on the
-  // tiled kernel). Scale blocks of 4 n rows by 64 2^m columns.
-  const int bws = block_w % 64 == 0 ? __builtin_ctz(block_w / 64) : 0;
-  if (M > 1 && block_w == 64 << bws && block_h % 4 == 0 && A && B && C &&
-      wide_fits(A, B, C, K)) {
+  const int route = fp8_route(M, N, K, block_h, block_w, A && B && C && wide_fits(A, B, C, K));
+  if (route < LIN_GEMV) {
     WideSeg s{};
     s.a = A; s.total_rows = M; s.w0 = B; s.s0 = scale_inv; s.bh = block_h;
-    s.bws = bws; s.N = N; s.K = K; s.out = C;
-    return launch_wide(WD_FP8, 0, wide_tile(WD_FP8, M, N, device_cus()), s, nullptr, 1, nullptr);
+    s.bws = __builtin_ctz(block_w / 64); s.N = N; s.K = K; s.out = C;
+    return launch_wide(WD_FP8, 0, route, s, nullptr, 1, nullptr);
   }
-  // decode-size batches with the loader's 128 x 128 blocks: the layer's
-  // unpacked-weight GEMV (one wave per four weight rows, 16-byte weight
-  // loads dequantized in registers), which streams B once per launch
-  if (block_h == 128 && block_w == 128 && M <= 64 && N % 128 == 0 &&
-      K % 128 == 0)
+  // (one wave per four weight rows, 16-byte weight loads dequantized in
+  // registers; B streamed once per four rows of A)
+  if (route == LIN_GEMV)
     return launch_gemv(0, 0, A, 0, 0, nullptr, 1, M, nullptr, nullptr, 1,
                        nullptr, B, scale_inv, nullptr, nullptr, N, K, nullptr,
                        0.f, C, nullptr);
@@ -210,20 +273,17 @@ int sllm_ds_fp4_gemm_packed_dev(float* o, const float* a, const void* packed,
                                 const void* scale_e8m0, int M, int N, int K,
                                 int block_w) {
   SLLM_REQUIRE(K % 2 == 0 && block_w > 0, "fp4 gemm: K even, block_w > 0");
-  // from two rows: the matrix cores (7168 -> 2048, us: one row 11.9 on the
-  // GEMV below, 14.6 there; four rows 21.9 / 15, 64 rows 286 / 43; 300 rows
-  // 772 on the tiled kernel, 69 there)
-  if (M > 1 && N > 0 && block_w == 32 && a && packed && scale_e8m0 && o &&
-      wide_fits(a, packed, o, K)) {
+  const int route = fp4_route(M, N, K, block_w, a && packed && scale_e8m0 && o &&
+                                                    wide_fits(a, packed, o, K));
+  if (route < LIN_GEMV) {
     WideSeg s{};
     s.a = a; s.total_rows = M; s.w0 = (const uint8_t*)packed; s.s0 = scale_e8m0;
     s.N = N; s.K = K; s.out = o;
-    return launch_wide(WD_FP4, 0, wide_tile(WD_FP4, M, N, device_cus()), s, nullptr, 1, nullptr);
+    return launch_wide(WD_FP4, 0, route, s, nullptr, 1, nullptr);
   }
-  // decode-size batches with 32-column scale blocks: the layer's
-  // unpacked-weight GEMV in its MXFP4 form (the same nibble order, E2M1
-  // values and 0x00 / 0xFF scale convention)
-  if (block_w == 32 && M <= 64 && K % 32 == 0 && N % 16 == 0)
+  // (the layer's MXFP4 form: the same nibble order, E2M1 values and 0x00 /
+  // 0xFF scale convention)
+  if (route == LIN_GEMV)
     return launch_gemv(1, 0, a, 0, 0, nullptr, 1, M, nullptr, nullptr, 1,
                        nullptr, (const uint8_t*)packed, scale_e8m0, nullptr,
                        nullptr, N, K, nullptr, 0.f, o, nullptr);

@@ -32,15 +32,21 @@ def test_fp32_rows(M, N, K):
     _check(q4.gemv_rows(a, w, 0, 1.0), a, w, 4, 4)
 
 
-@pytest.mark.parametrize("N,K", [(128, 128), (384, 1152), (128, 2048)])
-def test_quantized_one_row(N, K):
-    from sllm_amd import deepseek, fp8
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (1, 384, 1152), (2, 128, 2048), (3, 256, 2048),
+                                   (4, 9216, 1024), (4, 20480, 1024)])
+def test_quantized_few_rows(M, N, K):
+    from sllm_amd import _lib, deepseek, fp8
     rng = np.random.default_rng(N + K)
-    a = rng.standard_normal((1, K)).astype(np.float32)
+    gemv = [_lib.lib().sllm_linear_plan_query(f, M, N, K, 128, 32 if f else 128, 1) == 5
+            for f in (0, 1)]
+    assert any(gemv)
+    a = rng.standard_normal((M, K)).astype(np.float32)
     q = rng.integers(0, 256, (N, K), dtype=np.uint8)
     q[(q & 0x7F) == 0x7F] = 0x30
     s = (rng.random((N // 128, K // 128)) + 0.5).astype(np.float32)
-    _check(fp8.fp8_gemm(a, q, s), a, codecs.dequant_fp8_block(q, s), 16, 16)
+    if gemv[0]:
+        _check(fp8.fp8_gemm(a, q, s), a, codecs.dequant_fp8_block(q, s), 16, 16)
     p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
     sc = rng.integers(115, 130, (N, K // 32), dtype=np.uint8)
-    _check(deepseek.fp4_moe_linear(a, p, sc), a, codecs.dequant_fp4_block(p, sc), 16, 32)
+    if gemv[1]:
+        _check(deepseek.fp4_moe_linear(a, p, sc), a, codecs.dequant_fp4_block(p, sc), 16, 32)

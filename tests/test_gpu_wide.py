@@ -53,16 +53,26 @@ def test_fp4_linear(M, N, K):
     _check(deepseek.fp4_moe_linear(a, p, s), a, codecs.dequant_fp4_block(p, s))
 
 
-# two whole 128-wide K steps; a half last step, which one K wave sits out
-@pytest.mark.parametrize("K", [256, 320])
-def test_large_linear_takes_the_tall_tile(K):
-    from sllm_amd import fp8
-    rng = np.random.default_rng(5)
-    M, N = 500, 4100
+# each tile (16 x 16, 16 x 32, 32 x 64, 32 x 128, FP8 32 x 256 or MXFP4 64 x
+# 128) with ragged rows and columns; K of one step, a partial last step over
+# the K waves, more than the four steps of the unrolled loop
+@pytest.mark.parametrize("fp4", [0, 1])
+@pytest.mark.parametrize("tile,M,N", [(0, 10, 520), (1, 30, 4090), (2, 35, 4090), (3, 200, 4090),
+                                      (4, 500, 4090)])
+@pytest.mark.parametrize("K", [64, 320, 1088])
+def test_every_linear_tile(fp4, tile, M, N, K):
+    from sllm_amd import _lib, deepseek, fp8
+    assert _lib.lib().sllm_linear_plan_query(fp4, M, N, K, 128, 32 if fp4 else 128, 1) == tile
+    rng = np.random.default_rng(tile + K)
     a = rng.standard_normal((M, K)).astype(np.float32)
-    q = rng.integers(0, 0x70, (N, K), dtype=np.uint8)
-    s = (rng.random((-(-N // 128), -(-K // 128))) + 0.5).astype(np.float32)
-    _check(fp8.fp8_gemm(a, q, s), a, codecs.dequant_fp8_block(q, s))
+    if fp4:
+        p = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+        s = rng.integers(115, 130, (N, K // 32), dtype=np.uint8)
+        _check(deepseek.fp4_moe_linear(a, p, s), a, codecs.dequant_fp4_block(p, s))
+    else:
+        q = rng.integers(0, 0x70, (N, K), dtype=np.uint8)
+        s = (rng.random((-(-N // 128), -(-K // 128))) + 0.5).astype(np.float32)
+        _check(fp8.fp8_gemm(a, q, s), a, codecs.dequant_fp8_block(q, s))
 
 
 @pytest.mark.parametrize("M", [3, 40])

@@ -1,5 +1,5 @@
 """Which kernel and tile the host picks (no GPU needed): the bf16-weight
-layer."""
+layer, the FP8 and MXFP4 linears (at 256 CUs)."""
 import ctypes
 
 import pytest
@@ -75,3 +75,43 @@ def test_bf16_plan_rejects_bad_sizes():
     out = (ctypes.c_int * 4)()
     assert _lib.lib().sllm_moe_bf16_plan_query(4, 100, 8, 128, 0, 2, 1, out) == -1
     assert _lib.lib().sllm_moe_bf16_plan_query(4, 256, 8, 128, 0, 9, 1, out) == -1
+
+
+GEMV, TILED = 5, 6
+
+
+def _linear(fp4, M, N, K, bh=128, bw=None, aligned=1):
+    return _lib.lib().sllm_linear_plan_query(fp4, M, N, K, bh, bw or (32 if fp4 else 128), aligned)
+
+
+# rows that stream through the GEMV, rows from which the matrix cores run
+@pytest.mark.parametrize("fp4,N,K,gemv,wide", [
+    (0, 4096, 4096, (1, 2), (3, 64, 65)), (0, 7168, 2048, (2, 3), (4,)), (0, 2048, 7168, (1,), (2,)),
+    (0, 256, 256, (1,), (2,)), (0, 12288, 4096, (2, 4), (5,)), (0, 14336, 4096, (1,), (2,)),
+    (0, 17408, 5120, (2, 3), (4,)), (0, 151936, 2048, (2,), (3,)),
+    (1, 4096, 4096, (1, 2), (3,)), (1, 2048, 2048, (2, 3), (4,)), (1, 2048, 7168, (1,), (2,)),
+    (1, 256, 256, (1,), (2,)), (1, 18432, 7168, (2,), (3,)), (1, 20480, 2048, (2, 4), (5,)),
+    (1, 32000, 4096, (1,), (2,))])
+def test_linear_few_rows(fp4, N, K, gemv, wide):
+    for M in gemv:
+        assert _linear(fp4, M, N, K) == GEMV, M
+    for M in wide:
+        assert 0 <= _linear(fp4, M, N, K) < GEMV, M
+
+
+def test_linear_fallbacks():
+    """What the matrix-core kernel does not take: unaligned operands, a K
+    that is no multiple of 64, other scale blocks."""
+    assert _linear(0, 8, 256, 256, aligned=0) == GEMV
+    assert _linear(0, 80, 256, 256, aligned=0) == TILED
+    assert _linear(0, 8, 300, 200) == TILED        # ragged for both
+    assert _linear(0, 8, 256, 256, bh=6) == TILED  # block rows not in fours
+    assert _linear(0, 8, 256, 256, bw=192) == TILED
+    assert 0 <= _linear(0, 8, 256, 256, bh=4, bw=64) < GEMV
+    assert _linear(0, 1, 300, 256) == TILED        # one row off the 128 grid
+    assert _linear(1, 8, 256, 96) == GEMV
+    assert _linear(1, 80, 256, 96) == TILED
+    assert _linear(1, 8, 250, 96) == TILED
+    assert _linear(1, 2, 250, 256) < GEMV
+    assert _linear(1, 8, 256, 256, bw=16) == TILED
+    assert _linear(0, 0, 256, 256) == -1
