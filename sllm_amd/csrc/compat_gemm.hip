@@ -319,9 +319,9 @@ int sllm_ds_fp4_gemm_packed(float* o, const float* a, const void* packed,
 // and w (dtype tags of kernels/_sllm_cuda.py:490-491). Device pointers.
 // bf16 with k % 128 == 0 runs on the router GEMM kernels (the same contract:
 // bf16 products on the matrix cores, fp32 accumulation; m <= 64, the decode
-// loops' GEMVs, on the K-split small-batch kernel); other batches of at most
-// 64 rows (fp32, or bf16 with other k) on the unpacked-weight GEMV; the rest
-// on the tiled kernel.
+// loops' GEMVs, and few tiles of 64 x 128 at larger k on the K-split kernel,
+// the rest on the tiles); other batches of at most 64 rows (fp32, or bf16 with
+// other k) on the unpacked-weight GEMV; the rest on the tiled kernel.
 int sllm_gemm_ex(const void* a, int atype, const void* w, void* c, int m,
                  int n, int k) {
   SLLM_REQUIRE(atype == 0 || atype == 1, "sllm_gemm_ex: atype must be 0 or 1");
@@ -329,8 +329,8 @@ int sllm_gemm_ex(const void* a, int atype, const void* w, void* c, int m,
                "sllm_gemm_ex: null pointer or empty shape (m=%d n=%d k=%d)",
                m, n, k);
   if (atype == 1 && k % 128 == 0)
-    return launch_router_gemm((const uint16_t*)a, (const uint16_t*)w,
-                              (float*)c, m, n, k, nullptr, 1);
+    return launch_bf16_gemm((const uint16_t*)a, (const uint16_t*)w, (float*)c,
+                            m, n, k, nullptr);
   // other decode-size batches: the unpacked-weight GEMV (bf16 or fp32 rows)
   if (m <= 64 && n % 16 == 0 && k % (atype == 1 ? 8 : 4) == 0)
     return launch_gemv(atype == 1 ? 2 : 3, 0, a, atype, 0, nullptr, 1, m,

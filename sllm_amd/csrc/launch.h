@@ -17,10 +17,15 @@ bool router_short(int T, int E);
 // chunk histograms, which a softmax routing launch given them as
 // chunk_hist then fills (integer atomics: the counts do not depend on
 // order), so that launch_permute(..., hist_ready = true) skips its
-// histogram pass.
+// histogram pass. tiles: above 64 tokens the 64 x 128 tiles also where
+// router_short picks the K-split kernel.
 int launch_router_gemm(const uint16_t* x, const uint16_t* w, float* logits,
                        int T, int E, int H, hipStream_t st, int ks = 1,
-                       int* zero = nullptr, long zero_n = 0);
+                       int* zero = nullptr, long zero_n = 0, bool tiles = false);
+// c (m, n) fp32 = a (m, k) . w (n, k)^T in bf16 by the faster of the two
+// (k % 128 == 0): the standalone calls.
+int launch_bf16_gemm(const uint16_t* a, const uint16_t* w, float* c, int m,
+                     int n, int k, hipStream_t st);
 // Per-token activation quantization run by the softmax routing launch
 // (act_quant.h; x == nullptr: none).
 struct ActQuant {

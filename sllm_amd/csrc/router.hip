@@ -166,9 +166,9 @@ __global__ __launch_bounds__(512, 1) void router_gemm_kernel(
 }
 
 // Small T (decode, T <= 64; the few token tiles of a short prompt): a
-// workgroup owns 16 experts and up to 64 tokens (tile blockIdx.z); its 8 waves split K (wave w takes the 32-wide slices w, w + 8, ...) so the
-// router weights stream through many CUs at once; partial sums are reduced
-// through LDS.
+// workgroup owns 16 experts and up to 64 tokens (tile blockIdx.z); its 8 waves
+// split K (wave w takes the 32-wide slices w, w + 8, ...) so the router weights
+// stream through many CUs at once; partial sums are reduced through LDS.
 constexpr int RG_SMALL_T = 64;
 
 // Decode-size router GEMM: workgroup (x, q) computes experts [16 x, +16)
@@ -902,14 +902,26 @@ static int launch_router_small(const uint16_t* x, const uint16_t* w,
   return 0;
 }
 
+int launch_bf16_gemm(const uint16_t* a, const uint16_t* w, float* c, int m,
+                     int n, int k, hipStream_t st) {
+  // above 64 rows, where the tiles are few and unsplit: the K-split kernel is
+  // faster from K = 640 (us, tiles / K split, 512 x 512: K 256 4.5 / 5.4, 512
+  // 6.1 / 6.8, 640 6.9 / 6.8, 1024 8.9 / 6.8, 2048 15.1 / 11.1; 128 x 2048 x
+  // 7168 45.0 / 34.2; off 64 bits 2.7e-7 / 1.0e-7 at K = 2048), but for many
+  // rows of a wide product at K whose slices fill a wave's four loads badly
+  // (2048 x 128: K 1152 9.6 / 9.4, 1536 11.9 / 13.6, 1792 13.3 / 13.4)
+  const bool slow = k <= 512 || (m > 1280 && n > 64 && k > 1152 && k < 1792);
+  return launch_router_gemm(a, w, c, m, n, k, st, 1, nullptr, 0, slow);
+}
+
 int launch_router_gemm(const uint16_t* x, const uint16_t* w, float* logits,
                        int T, int E, int H, hipStream_t st, int ks,
-                       int* zero, long zero_n) {
+                       int* zero, long zero_n, bool tiles) {
   SLLM_REQUIRE(x && w && logits, "router_gemm: null pointer");
   SLLM_REQUIRE(T > 0 && E > 0 && H > 0 && H % 128 == 0,
                "router_gemm: need T,E>0 and H %% 128 == 0 (T=%d E=%d H=%d)",
                T, E, H);
-  const bool small = T <= RG_SMALL_T || router_short(T, E);
+  const bool small = T <= RG_SMALL_T || (router_short(T, E) && !tiles);
   SLLM_REQUIRE(ks == 1 || small, "router_gemm: K split of T=%d E=%d", T, E);
   SLLM_REQUIRE(zero_n == 0 || zero, "router_gemm: null zero range");
   if (small) {
@@ -1233,8 +1245,8 @@ int sllm_q4_moe_router_dev(const float* logits, float* w_out, int* id_out,
 
 int sllm_moe_router_gemm(const void* x_bf16, const void* w_bf16,
                          float* logits, int T, int E, int H, void* stream) {
-  return launch_router_gemm((const uint16_t*)x_bf16, (const uint16_t*)w_bf16,
-                            logits, T, E, H, (hipStream_t)stream);
+  return launch_bf16_gemm((const uint16_t*)x_bf16, (const uint16_t*)w_bf16,
+                          logits, T, E, H, (hipStream_t)stream);
 }
 
 int sllm_moe_route_softmax(const float* logits, float* w_out, int* id_out,

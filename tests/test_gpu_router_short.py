@@ -47,3 +47,26 @@ def test_deepseek_short_prompt_router(T, H):
     np.testing.assert_array_equal(r["w"], r_g["w"])
     np.testing.assert_array_equal(y, y_g)
     np.testing.assert_array_equal(layer.forward(x, mode="prefill"), y)
+
+
+# bf16 gemm_ex above 64 rows: the K-split kernel (a few 64 x 128 tiles, K from
+# 640; one to four slices a wave, a partial round), the tiles at shorter K, at
+# many rows with K 1280, and past 32 tiles
+@pytest.mark.parametrize("m,n,k", [
+    (65, 200, 640), (300, 129, 1024), (1290, 100, 1152), (70, 2000, 1792), (2048, 16, 1408),
+    (300, 129, 512), (1290, 100, 1280), (2049, 70, 1664), (330, 770, 1024)])
+def test_bf16_gemm_both_kernels(m, n, k):
+    """Products of bf16 values are exact in fp32; each of the K / 32 MFMA
+    steps adds 32 of them with a few roundings, the K-split kernel's waves
+    once more: |error| <= (K / 32 * 6 + 8) 2^-24 sum |a w|."""
+    from oracle import codecs
+    from sllm_amd.runtime import DeviceBuffer, T_BF16, gemm_ex, sync, to_bf16, to_device_raw
+    rng = np.random.default_rng(m * n + k)
+    a = codecs.round_bf16(rng.standard_normal((m, k)).astype(np.float32))
+    w = codecs.round_bf16(rng.standard_normal((n, k)).astype(np.float32))
+    c = DeviceBuffer(m * n * 4)
+    gemm_ex(to_device_raw(to_bf16(a)), to_device_raw(to_bf16(w)), c, m, n, k, T_BF16)
+    sync()
+    want = a.astype(np.float64) @ w.astype(np.float64).T
+    mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert np.all(np.abs(c.copy_host().reshape(m, n) - want) <= (k / 32 * 6 + 8) * 2.0 ** -24 * mag)
