@@ -4,9 +4,10 @@
 // plain or as a SwiGLU pair, for one matrix or for a layer's row tiles.
 //
 // Serves the bf16-weight MoE layer (moe_layer.hip) and the standalone FP8
-// and MXFP4 linears (compat_gemm.hip) at the sizes where the per-wave GEMV
-// (decode.hip), which multiplies on the vector ALU and passes over the
-// weights once per four rows, is not bound by the weight stream any more.
+// and MXFP4 linears (compat_gemm.hip) from the few rows on at which the
+// per-wave GEMV (decode.hip), which multiplies on the vector ALU and passes
+// over the weights once per four rows, is not bound by the weight stream any
+// more (bf16_gemv, fp8_few_rows, fp4_few_rows).
 //
 // fp32 precision on bf16 MFMAs. An fp32 activation, times a power of two, is
 // the exact sum of three bf16 values, its significand cut in 8 + 8 + 8 bits
@@ -27,17 +28,20 @@
 // lane's load 16 or 32 contiguous bytes (lane group g takes K [16 g, +16) of
 // a 64-wide step for both operands).
 //
-// What bounds it: vector ALU issue beside the MFMAs (the split, 5
-// instructions an element, is repeated by every column tile; the FP8
-// conversion one per two weights), two waves a SIMD. FP8 512 x 4096 x 4096:
-// 738 us on the tiled kernel, 54 here (0.95 PFLOP/s of bf16 products, the
-// product itself 317 TFLOP/s); 32 rows 76 -> 13 us. MXFP4 300 x 2048 x 7168:
-// 772 -> 69 us. bf16 layer (H 1024, E 16, I 512, top-4): 64 tokens 212 -> 43
-// us, 1000 tokens 2712 -> 110 us, there by the L2's rate: a tile's K step
-// brings its rows of both operands in (32 x 128 tiles: 153 us). Against 64
-// bits the error is below that of the GEMV (layer 1.5e-7 to 1.8e-7 up to 64
-// tokens) and of the tiled kernel (linears 1.3e-7 and 1.6e-7, there 1.1e-6 and
-// 1.4e-6).
+// What bounds it: latency, with two waves a SIMD and a barrier a step. Of the
+// cycles of an FP8 512 x 4096 x 4096 launch the matrix cores are busy in 24%
+// and the vector ALU in 22% (the split, 4.5 instructions an element, is
+// repeated by every column tile; the FP8 conversion one per two weights), the
+// waves wait for 44% of their time, LDS conflicts take 6%; MXFP4 300 x 2048 x 7168
+// 15, 18, 28 and 7% with 160 workgroups on 256 CUs; the bf16 layer's gate/up at
+// 1000 tokens 9, 12, 43 and 4%, 64% L2 hits. FP8 512 x 4096 x 4096: 738 us on
+// the tiled kernel, 54 here (0.95 PFLOP/s of bf16 products, the product itself
+// 317 TFLOP/s); 32 rows 67 -> 12 us. MXFP4 300 x 2048 x 7168: 772 -> 67 us. bf16
+// layer (H 1024, E 16, I 512, top-4, a shared expert): 64 tokens 212 -> 43 us,
+// 1000 tokens 2712 -> 108 us (32 x 128 tiles: 153 us). Against 64 bits the error
+// is below that of the tiled kernel (linears 1.3e-7 and 1.6e-7, there 1.1e-6 and
+// 1.4e-6) and of the GEMV with fp32 wave sums that it was measured against
+// (layer 1.5e-7 to 1.8e-7 up to 64 tokens).
 #include "launch.h"
 
 namespace sllm {
@@ -77,8 +81,8 @@ constexpr int A_UP = 40;
 
 // Two fp32 values, scaled, as three bf16 pairs each cut off (truncated) in
 // turn: hi + mid + lo is the value exactly (8 + 8 + 8 significand bits). An
-// infinity or NaN, or a value past 2^88, gives its row's sums infinities or
-// NaN, which are taken again.
+// infinity or NaN, or a value past 2^88 (or of less, whose products are past
+// it), gives its row's sums infinities or NaN, which are taken again.
 __device__ __forceinline__ void split3(float a, float b, uint32_t m1lo,
                                        uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   constexpr float UP = (float)(1ull << A_UP);
@@ -91,7 +95,7 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t m1lo,
 }
 
 // e4m3 is exact in bf16; v_cvt_scalef32_pk_bf16_fp8 at scale 1 converts two
-// bytes (checked on gfx950 against the fp32 conversion for every byte pair)
+// bytes (every pair of finite codes is tested)
 __device__ __forceinline__ bf16x8 e4m3x8(uint32_t d0, uint32_t d1) {
   const u32x4 r = {
       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d0, 1.f, false)),
@@ -191,7 +195,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   constexpr int NW = WBytes<WF>::regs;
   static_assert(NA >= 1 && NA * CE * WD_THREADS == BM * KT, "whole chunks");
   // gate/up up to 32-row tiles: the K steps' sum keeps its rounding errors
-  // beside it. Layer against 64 bits at 64 tokens, H 1024 / 2048: 1.64e-7 /
+  // beside it (of each step whose partial is below the sum, most of it else:
+  // the two-operand form). Layer against 64 bits at 64 tokens, H 1024 / 2048: 1.64e-7 /
   // 1.98e-7 without (the GEMV 1.60e-7 / 1.82e-7), 1.48e-7 / 1.69e-7 with it, for 1
   // to 3% of the layer's time (41.9 -> 42.9 us, 104 -> 106); in the down launch
   // too 1.46e-7 / 1.64e-7 for twice that. 64-row tiles are below the GEMV that
@@ -209,7 +214,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   const int b = second ? blockIdx.x - blocks0 : blockIdx.x;
   const int NS = (S.N + BN - 1) / BN;
   // column slabs vary fastest: with a multiple of eight of them a slab's row
-  // tiles run on one XCD and share its weights in that L2
+  // tiles run on one XCD and share its weights in that L2 (with four, as the
+  // bf16 layer's gate/up at I 512, on two)
   const int rt = b / NS, ns = b % NS;
   int e = 0, rb0 = rt * BM, rows;
   if (S.tile_info) {
@@ -555,28 +561,32 @@ int go(const WideSeg& s0, const WideSeg& s1, int topk, hipStream_t st) {
 
 }  // namespace
 
-// The linears' tiles (rows x output columns) and the time of one of their
+// The linears' tiles (rows x output columns) and the time of a round of their
 // workgroups in us at K = 4096, FP8 and MXFP4 weights, by which wide_tile
-// weighs them.
+// weighs them (a launch of one to three rounds over N = 4096, divided by them;
+// MXFP4's shortest tiles at a few rows, which cost less than sixteen).
 struct WideTile {
   int bm, bn;
   float us;
 };
 static const WideTile WIDE_FP8[] = {
-    {16, 16, 12.f}, {16, 32, 12.7f}, {32, 64, 23.f}, {32, 128, 33.5f}, {32, 256, 50.f}};
+    {16, 16, 11.5f}, {16, 32, 12.4f}, {32, 64, 22.f}, {32, 128, 31.5f}, {32, 256, 52.f}};
 static const WideTile WIDE_FP4[] = {
     {16, 16, 9.5f}, {16, 32, 12.5f}, {32, 64, 23.8f}, {32, 128, 39.f}, {64, 128, 64.f}};
 
 // One workgroup fits a CU (its registers and tile), so a launch takes as
 // many rounds as its tiles need over the CUs. FP8 4096 x 4096, us by tile:
-// 16 rows 11.8 / 12.4 / 23 / 34 / 54, 32 rows 21.7 / 12.7 / 23 / 34 / 55, 256
-// rows - / - / 50 / 36 / 55, 512 rows - / - / 93 / 68 / 54 (64 x 128, which
-// spills there: 62). The tallest FP8 tile is four waves of 64 columns by two
-// K halves: an LDS fragment serves four products, not two, and half as many
-// barriers follow (eight waves of 32 columns: 300 / 400 / 512 rows 54.7 / 55.9 /
-// 57.4 us, so 51.3 / 51.9 / 54.1). MXFP4, whose conversions that form holds
-// in registers too, keeps 64 x 128 (7168 <- 2048, 150 / 222 / 512 rows 37.3 /
-// 38.4 / 76.0 us there, 44.0 / 44.9 / 88.1 as 32 x 256).
+// 16 rows 11.5 / 12.4 / 21 / 30 / 48, 32 rows 21.4 / 13.0 / 22 / 31 / 49, 128 rows
+// 75 / 44 / 22.3 / 30.7 / 50, 256 rows - / 86 / 43 / 32.9 / 51, 512 rows - / - / 84 /
+// 63.2 / 54.6, 513 and 768 rows (three rounds, or two) 90.4 / 98.1 and 94.2 /
+// 100.9 of the last two, 1024 rows 125 / 106; 64 x 128 as the tallest spilled 62 at
+// 512. The tallest FP8 tile is four waves of 64 columns by two K halves: an
+// LDS fragment serves four products, not two, and half as many barriers
+// follow (eight waves of 32 columns: 300 / 400 / 512 rows 54.7 / 55.9 / 57.4 us, so
+// 51.3 / 51.9 / 54.1); it holds all 256 registers and spills five. MXFP4, whose
+// conversions that form holds in registers too, keeps 64 x 128 (7168 <- 2048,
+// 150 / 222 / 512 rows 37.3 / 38.4 / 76.0 us there, 44.0 / 44.9 / 88.1 as 32 x
+// 256).
 int wide_tile(int wf, long rows, long n, int num_cus) {
   const WideTile* tile = wf == WD_FP8 ? WIDE_FP8 : WIDE_FP4;
   int best = 0;

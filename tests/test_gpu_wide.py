@@ -101,6 +101,21 @@ def test_nonfinite_activations(M):
     assert np.all(np.isfinite(np.delete(y, 4, 1)))
 
 
+def test_every_pair_of_fp8_codes():
+    """One-hot activations read the converted weights back: every pair of
+    finite codes, in either half of a dword, exactly."""
+    from sllm_amd import fp8
+    K, N = 64, 2048
+    codes = np.arange(65536, dtype=np.uint32)
+    q = np.stack([codes & 255, codes >> 8], -1).astype(np.uint8)
+    q[(q & 0x7F) == 0x7F] = 0
+    for q2 in (q, np.roll(q, 1, axis=0)):  # (each pair in the other half)
+        w = q2.reshape(N, K)
+        got = fp8.fp8_gemm(np.eye(K, dtype=np.float32), w, np.ones((N // 128, 1), np.float32),
+                           128, 64)
+        np.testing.assert_array_equal(got, codecs.decode_e4m3fn(w).T)
+
+
 def _product(a, wd):
     """The fp64 product with what 0 and infinities give (an fp32 overflow as
     an infinity)."""

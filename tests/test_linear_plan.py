@@ -99,6 +99,14 @@ def test_linear_few_rows(fp4, N, K, gemv, wide):
         assert 0 <= _linear(fp4, M, N, K) < GEMV, M
 
 
+def test_fp8_tile_by_rounds():
+    """4096 columns: 32 x 256 tiles for a full round and an even number of
+    them, 32 x 128 in between."""
+    for M, tile in ((16, 0), (32, 1), (128, 2), (256, 3), (300, 4), (512, 4), (513, 3), (768, 3),
+                    (1000, 4), (1024, 4)):
+        assert _linear(0, M, 4096, 4096) == tile, M
+
+
 def test_linear_fallbacks():
     """What the matrix-core kernel does not take: unaligned operands, a K
     that is no multiple of 64, other scale blocks."""
