@@ -519,7 +519,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
 #pragma unroll
     for (int i = 0; i < RB * NC * 4; ++i)
       z = fmaf(acc[i / (4 * NC)][i / 4 % NC][i % 4], 0.f, z);
-    if (!__ballot(z != 0.f)) return;
+    // (rows that a 16-row tile leaves unstaged hold anything)
+    if (!__ballot(z != 0.f && (RB > 1 || lc < rows))) return;
     uint32_t bad = 0;
 #pragma unroll
     for (int i = 0; i < RB * NC * 4; ++i) {
