@@ -512,7 +512,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   // FP8 partial that overflows before a small block scale, or an infinite
   // weight (a bf16 one, e8m0 254) against a zero mid or lo part. Those
   // outputs are taken again by plain fp32 products, an output at a time by
-  // the whole wave (its weights laid out as the loads above read them).
+  // the whole wave (its weights laid out as the loads above read them). A row
+  // that holds a NaN is NaN throughout: left as it is after one of them.
   if constexpr (A32) {
     static_assert(RB * NC * 4 <= 32, "a bit for each of a lane's sums");
     float z = 0.f;
@@ -529,16 +530,28 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
           !__builtin_isfinite(acc[r][c][v]))
         bad |= 1u << i;
     }
+    uint64_t seen = 0;  // rows looked over for a NaN
     while (const uint64_t m = __ballot(bad != 0)) {
       const int l = __builtin_ctzll(m);
       const int i = __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)bad, l));
       const int t = i / (4 * NC) * 16 + (l & 15), p = rb0 + t;
       const int n = ncol + i / 4 % NC * 16 + 4 * (l >> 4) + i % 4;
-      float y = plain_dot<WF>(S, (const float*)S.a + (size_t)rsrc[t] * K, e, n, lane);
+      const float* a = (const float*)S.a + (size_t)rsrc[t] * K;
+      float y = plain_dot<WF>(S, a, e, n, lane);
+      if (__builtin_isnan(y) && !(seen >> t & 1)) {
+        seen |= 1ull << t;
+        bool nan = false;
+        for (int k = 4 * lane; k < K; k += 256) {
+          const float4 v = *(const float4*)(a + k);
+          nan |= __builtin_isunordered(v.x, v.y) || __builtin_isunordered(v.z, v.w);
+        }
+        if (__any(nan) && lc == (l & 15))
+          bad &= ~(((1u << (4 * NC - 1) << 1) - 1) << (i / (4 * NC) * 4 * NC));
+      }
       if (S.row_w) y *= S.row_w[S.sorted_idx ? S.sorted_idx[p] : p];
       if (lane == l) {
         S.out[(size_t)p * N + n] = y;
-        bad &= bad - 1;
+        bad &= ~(1u << i);
       }
     }
   }

@@ -101,6 +101,30 @@ def test_nonfinite_activations(M):
     assert np.all(np.isfinite(np.delete(y, 4, 1)))
 
 
+def test_nonfinite_rows_of_a_tall_tile():
+    """NaN, infinite and overflowing rows of one 32-row tile beside each
+    other: each row as a plain product has it, the finite ones untouched."""
+    from sllm_amd import _lib, fp8
+    M, N, K = 500, 4090, 128
+    assert _lib.lib().sllm_linear_plan_query(0, M, N, K, 128, 128, 1) == 4
+    rng = np.random.default_rng(7)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    q = rng.integers(0x20, 0x70, (N, K), dtype=np.uint8)
+    q[::3] |= 0x80
+    q[5, 9] = 0
+    s = np.full((-(-N // 128), 1), 1e-3, np.float32)
+    clean = fp8.fp8_gemm(a, q, s)
+    a[3, 7], a[19, 100], a[35, 9], a[50] = np.nan, np.inf, -np.inf, 3e37
+    a[51, 0], a[51, 1] = np.inf, -np.inf
+    got = fp8.fp8_gemm(a, q, s)
+    wd = codecs.dequant_fp8_block(q, s)
+    for m in (3, 19, 35, 51):
+        np.testing.assert_array_equal(got[m], _product(a[m:m + 1], wd)[0])
+    _check(got[50:51], a[50:51], wd)
+    keep = np.setdiff1d(np.arange(M), (3, 19, 35, 50, 51))
+    np.testing.assert_array_equal(got[keep], clean[keep])
+
+
 def test_every_pair_of_fp8_codes():
     """One-hot activations read the converted weights back: every pair of
     finite codes, in either half of a dword, exactly."""
