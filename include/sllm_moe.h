@@ -319,8 +319,10 @@ typedef struct sllm_moe_qwen_args {
   int mode;
   int out_f32;
   int logits_given;
-  int wdtype; /* 0: FP8 e4m3 + fp32 block scales; 1: bf16 (scales unused,
-                 always the fp32-activation GEMV path) */
+  int wdtype; /* 0: FP8 e4m3 + fp32 block scales; 1: bf16 (scales unused;
+                 unquantized activations at every T: the matrix-core kernel,
+                 or with few rows an expert or weights off 16 bytes the GEMV:
+                 sllm_moe_bf16_plan_query) */
   float renorm_eps;
   const void* x;
   const float* logits;

@@ -456,9 +456,10 @@ int launch_gemv(int wf, int swiglu, const void* act, int act_bf16,
 // (s1 may be null) of equal format. tile: the workgroup's rows x columns, 0
 // 16 x 16, 1 16 x 32, 2 32 x 64, 3 32 x 128, 4 32 x 256 (FP8), 64 x 128
 // (MXFP4) or 64 x 256 (bf16); swiglu: half the columns of 1-4; wide_tile
-// picks the linears'; tile_info rows must fit. K a
-// multiple of 64 (and 16-byte aligned pointers): wide_fits; FP8: bh a
-// multiple of 4.
+// picks the linears'; tile_info rows must fit. K a multiple of 64 (and 16-byte
+// aligned pointers): wide_fits; FP8: bh a multiple of 4. A, weights and scales
+// of any value: what a plain fp32 product of the scaled weight gives, to the
+// rounding of its sums, also where it is infinite or NaN.
 enum { WD_BF16 = 0, WD_FP8 = 1, WD_FP4 = 2 };
 struct WideSeg {
   const void* a;          // rows, stride K; null: no segment

@@ -612,8 +612,8 @@ def moe_block_forward(x, router_w, expert_gate, expert_up, expert_down,
                       shared_gate_w, shared_gate_linear_w, shared_up_w,
                       shared_down_w, top_k, eps=1e-20):
     """Device twin of ref/qwen4_exp.py:153-184 moe_block_forward with the
-    same signature: weights are float arrays used at bf16 precision (the
-    bf16 GEMV path, fp32 activations). Returns (n, H) float32.
+    same signature: weights are float arrays used at bf16 precision,
+    activations unquantized. Returns (n, H) float32.
 
     The device layer (weights uploaded once) is kept between calls with the
     same weights (see BLOCK_CACHE_MAX); any hidden and intermediate sizes

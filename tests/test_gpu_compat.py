@@ -103,9 +103,9 @@ def test_fp8_gemm_scale_orientation():
 
 @pytest.mark.parametrize("M,N,K", [(1, 256, 512), (33, 384, 1024), (64, 128, 128)])
 def test_fp8_gemm_decode_shapes(M, N, K):
-    """sllm_fp8_gemm at decode sizes with 128 x 128 blocks (M <= 64, N and K
-    multiples of 128: the unpacked-weight GEMV path) against the fp64
-    product with the dequantized weight."""
+    """sllm_fp8_gemm at decode sizes with 128 x 128 blocks (N and K multiples
+    of 128; one row on the unpacked-weight GEMV, more on the matrix-core
+    kernel) against the fp64 product with the dequantized weight."""
     from sllm_amd import fp8
     rng = np.random.default_rng(M + N + K)
     a = rng.standard_normal((M, K)).astype(np.float32)
@@ -183,8 +183,9 @@ def test_fp4_linear_matches_dequant():
 
 @pytest.mark.parametrize("M,N,K", [(1, 256, 512), (40, 128, 1024), (64, 48, 96)])
 def test_fp4_linear_decode_shapes(M, N, K):
-    """Packed MXFP4 linear at decode sizes (M <= 64, 32-column scale blocks:
-    the unpacked-weight GEMV path), including e8m0 scale codes 0 (-> 0)
+    """Packed MXFP4 linear at decode sizes (32-column scale blocks; one row,
+    and K 96, on the unpacked-weight GEMV, 40 rows on the matrix-core
+    kernel), including e8m0 scale codes 0 (-> 0)
     and 255 (-> NaN, a NaN row), against the fp64 product."""
     from sllm_amd import deepseek
     rng = np.random.default_rng(M * N + K)
@@ -247,8 +248,8 @@ def test_gemm_ex_gemv_shapes(atype, m, n, k):
                                    (65, 200, 384), (300, 129, 1024)])
 def test_gemm_ex_bf16_mfma_shapes(m, n, k):
     """bf16 gemm_ex with k % 128 == 0 (the MFMA router kernels: the K-split
-    small-batch kernel for m <= 64, the 64 x 128 tiles above; ragged n and
-    m): against the fp64 product of the bf16-rounded operands. bf16 products
+    small-batch kernel for m <= 64 and for few tiles at k 1024, the 64 x 128
+    tiles at 65 rows and k 384; ragged n and m): against the fp64 product of the bf16-rounded operands. bf16 products
     are exact in fp32, so only the fp32 accumulation order differs."""
     from sllm_amd.runtime import DeviceBuffer, T_BF16, gemm_ex, sync, to_bf16, to_device_raw
     rng = np.random.default_rng(m * n + k)
