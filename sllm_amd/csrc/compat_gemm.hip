@@ -164,7 +164,7 @@ bool fp4_few_rows(int M, int N, int K, int cus) {
 }
 
 // FP8: the matrix cores take scale blocks of 4 n rows by 64 2^m columns, the
-// GEMV the loader's 128 x 128. fits: wide_fits and no null pointer.
+// GEMV the loader's 128 x 128. fits: wide_fits.
 int fp8_route(int M, int N, int K, int bh, int bw, bool fits) {
   const int cus = device_cus();
   const bool gemv = bh == 128 && bw == 128 && M <= 64 && N % 128 == 0 && K % 128 == 0;
@@ -205,8 +205,8 @@ int sllm_fp8_gemm_dev(const float* A, const unsigned char* B,
                       int block_h, int block_w) {
   SLLM_REQUIRE(M > 0 && N > 0 && K > 0 && block_h > 0 && block_w > 0,
                "sllm_fp8_gemm: bad dims");
-  SLLM_REQUIRE(scale_inv, "sllm_fp8_gemm: null scale");
-  const int route = fp8_route(M, N, K, block_h, block_w, A && B && C && wide_fits(A, B, C, K));
+  SLLM_REQUIRE(A && B && scale_inv && C, "sllm_fp8_gemm: null pointer");
+  const int route = fp8_route(M, N, K, block_h, block_w, wide_fits(A, B, C, K));
   if (route < LIN_GEMV) {
     WideSeg s{};
     s.a = A; s.total_rows = M; s.w0 = B; s.s0 = scale_inv; s.bh = block_h;
@@ -273,8 +273,8 @@ int sllm_ds_fp4_gemm_packed_dev(float* o, const float* a, const void* packed,
                                 const void* scale_e8m0, int M, int N, int K,
                                 int block_w) {
   SLLM_REQUIRE(K % 2 == 0 && block_w > 0, "fp4 gemm: K even, block_w > 0");
-  const int route = fp4_route(M, N, K, block_w, a && packed && scale_e8m0 && o &&
-                                                    wide_fits(a, packed, o, K));
+  SLLM_REQUIRE(M <= 0 || (a && packed && scale_e8m0 && o), "fp4 gemm: null pointer");
+  const int route = fp4_route(M, N, K, block_w, wide_fits(a, packed, o, K));
   if (route < LIN_GEMV) {
     WideSeg s{};
     s.a = a; s.total_rows = M; s.w0 = (const uint8_t*)packed; s.s0 = scale_e8m0;

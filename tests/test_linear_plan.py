@@ -123,3 +123,15 @@ def test_linear_fallbacks():
     assert _linear(1, 2, 250, 256) < GEMV
     assert _linear(1, 8, 256, 256, bw=16) == TILED
     assert _linear(0, 0, 256, 256) == -1
+
+
+@pytest.mark.parametrize("hole", [0, 1, 2, 3])
+def test_linears_refuse_null_pointers(hole):
+    """Before any launch, at every batch size."""
+    lib = _lib.lib()
+    for M in (1, 8, 80):
+        p = [ctypes.c_void_p(0 if i == hole else 4096) for i in range(4)]
+        assert lib.sllm_fp8_gemm_dev(*p, M, 128, 128, 128, 128) == -1
+        assert "null" in _lib.last_error()
+        assert lib.sllm_ds_fp4_gemm_packed_dev(*p, M, 128, 128, 32) == -1
+        assert "null" in _lib.last_error()
