@@ -16,9 +16,10 @@
 // that contract; the contract is what is implemented.
 //
 // FP8 and MXFP4 weights of the loader's block shapes run on the matrix cores
-// (gemm_wide.hip), bf16 gemm_ex with k % 128 == 0 on the MFMA router kernels;
-// other shapes take a 32x32 LDS-tiled fp32 kernel with on-the-fly
-// dequantization of B.
+// (gemm_wide.hip) or, with few rows, on the layer's unpacked-weight GEMV
+// (decode.hip), bf16 gemm_ex with k % 128 == 0 on the MFMA router kernels;
+// other shapes take the GEMV up to 64 rows where it fits, else a 32x32
+// LDS-tiled fp32 kernel with on-the-fly dequantization of B.
 #include "launch.h"
 
 namespace sllm {

@@ -197,7 +197,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
   // gate/up up to 32-row tiles: the K steps' sum keeps its rounding errors
   // beside it (of each step whose partial is below the sum, most of it else:
   // the two-operand form). Layer against 64 bits at 64 tokens, H 1024 / 2048: 1.64e-7 /
-  // 1.98e-7 without (the GEMV 1.60e-7 / 1.82e-7), 1.48e-7 / 1.69e-7 with it, for 1
+  // 1.98e-7 without (the GEMV with fp32 wave sums 1.60e-7 / 1.82e-7, now 1.20e-7
+  // with 64-bit ones), 1.48e-7 / 1.69e-7 with it, for 1
   // to 3% of the layer's time (41.9 -> 42.9 us, 104 -> 106); in the down launch
   // too 1.46e-7 / 1.64e-7 for twice that. 64-row tiles are below the GEMV that
   // they replaced without it (1.82e-7 against 1.84e-7, 2.3e-7 against 3.6e-7).
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(WideSeg S0, WideSeg S1
     f32x4 part[RB][NC];
     // Fragments are read PL RB units ahead. bf16 weights take both K halves'
     // low parts first, so that the sums round while they are small (64-token
-    // layer 1.7e-7 -> 1.6e-7 off 64 bits, the GEMV's); the converted formats,
+    // layer 1.7e-7 -> 1.6e-7 off 64 bits); the converted formats,
     // which would hold both halves' weights for it (512 x 4096 x 4096 58.9 ->
     // 61.8 us), one K half after the other.
     constexpr int U = PL * RB;  // fragments of a K half; 2 U in all
